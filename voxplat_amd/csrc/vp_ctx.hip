@@ -30,7 +30,11 @@ int ensure_frame(vp_ctx *ctx, uint64_t pixels)
     // allocation leaves the old (smaller) pair and its capacities in place
     uint64_t *p = nullptr;
     float4 *r = nullptr;
-    if (hipMalloc(&p, pixels * sizeof(uint64_t)) != hipSuccess) return VP_ERR_NOMEM;
+    // the frame keys, then a 32-bit depth bound per 8x8 pixels: at most
+    // (w/8 + 1)(h/8 + 1) <= pixels/64 + pixels/8 + 2 of them for any w h = pixels
+    const uint64_t tiles = pixels / 64 + pixels / 8 + 2;
+    if (hipMalloc(&p, pixels * sizeof(uint64_t) + tiles * sizeof(uint32_t)) != hipSuccess)
+        return VP_ERR_NOMEM;
     if (hipMalloc(&r, pixels * sizeof(float4)) != hipSuccess) {
         (void)hipFree(p);
         return VP_ERR_NOMEM;
@@ -56,8 +60,9 @@ int ensure_blocks(vp_ctx *ctx, uint64_t blocks)
 {
     if (blocks <= ctx->blk_cap) return VP_OK;
     uint32_t *p = nullptr;
-    // a bin and an order slot per block, then 2 * 256 bin counters and the total
-    if (hipMalloc(&p, (2 * blocks + 2 * 256 + 1) * sizeof(uint32_t)) != hipSuccess)
+    // a screen box (4 words), a bin and an order slot per block, then 2 * 256
+    // bin counters and the total
+    if (hipMalloc(&p, (6 * blocks + 2 * 256 + 1) * sizeof(uint32_t)) != hipSuccess)
         return VP_ERR_NOMEM;
     if (ctx->d_blk) {
         if (hipDeviceSynchronize() != hipSuccess) return VP_ERR_HIP;

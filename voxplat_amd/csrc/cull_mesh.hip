@@ -122,8 +122,8 @@ struct Lay : Rows<B, V2> {
     static constexpr int mini(int a, int b) { return a < b ? a : b; }
     static constexpr int EB = MIP ? 2 : 4;
     static constexpr int LCAP = mini(MIP ? 1920 : 512, P::N0 * P::N0);
-    static constexpr int SWIN = 2 * P::R + 2;
-    static constexpr int WAVE_WORDS = (EB * LCAP + 2 * SWIN + 7) / 8;
+    static constexpr int SWIN = 2 * P::R + 1;    // bytes: one per map entry pair
+    static constexpr int WAVE_WORDS = (EB * LCAP + SWIN + 7) / 8;
     static constexpr int WAVES = SOFF + SOFF_WORDS;
     static constexpr int COL = WAVES + NW * WAVE_WORDS;
     // the +x neighbour's x = 0 plane as bytes, voxel (0, y, z) at z R + y:
@@ -177,25 +177,6 @@ __device__ __forceinline__ uint32_t rank_below(uint64_t m)
                                      __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
-// position of the k-th set bit (k counted from 0) of v; v has more than k bits
-__device__ __forceinline__ int select64(uint64_t v, uint32_t k)
-{
-    int pos = 0;
-    uint32_t c = __popc((uint32_t)v);
-    if (k >= c) { k -= c; v >>= 32; pos += 32; }
-    c = __popc((uint32_t)v & 0xFFFFu);
-    if (k >= c) { k -= c; v >>= 16; pos += 16; }
-    c = __popc((uint32_t)v & 0xFFu);
-    if (k >= c) { k -= c; v >>= 8; pos += 8; }
-    c = __popc((uint32_t)v & 0xFu);
-    if (k >= c) { k -= c; v >>= 4; pos += 4; }
-    c = __popc((uint32_t)v & 0x3u);
-    if (k >= c) { k -= c; v >>= 2; pos += 2; }
-    c = (uint32_t)v & 1u;
-    if (k >= c) pos += 1;
-    return pos;
-}
-
 struct ChunkRefs {
     const uint8_t *own, *nb[3];   // nb[a] == nullptr beyond the world
     int own_u, nb_u[3];           // uniform value or -1
@@ -221,6 +202,16 @@ __device__ __forceinline__ uint4 ld16(__amdgpu_buffer_rsrc_t rs, uint32_t voff, 
     typedef unsigned int v4u __attribute__((ext_vector_type(4)));
     const v4u v = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)voff, (int)soff, 0);
     return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+// 8 bytes at voff of the descriptor's range, non-temporal (the kernel never
+// reads its records back); lanes past the range store nothing.
+__device__ __forceinline__ void st8_nt(__amdgpu_buffer_rsrc_t rs, uint32_t voff, uint32_t lo,
+                                       uint32_t hi)
+{
+    typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+    const v2u v = {lo, hi};
+    __builtin_amdgcn_raw_buffer_store_b64(v, rs, (int)voff, 0, 2);
 }
 
 // Fill `dst` (row words, rowcount rows of R bits) from R-byte rows at src with
@@ -406,66 +397,26 @@ __device__ __forceinline__ uint32_t face_flags(const uint64_t *lds, int x, int y
     return f;
 }
 
-__device__ __forceinline__ uint32_t shadow_bit(const uint16_t *map, uint32_t sx, uint32_t wx,
-                                               uint32_t wy, uint32_t wz)
-{
-    if (!map) return 0u;
-    const uint32_t i = (wx + wy) + sx * wz;        // shadow.h:45-51, u32 wrap
-    return !(map[i] <= wy && map[i + 1] <= wy);    // shadow.h:54-63
-}
-
-template <bool V2>
-__device__ __forceinline__ uint64_t pack_record(uint32_t wx, uint32_t wy, uint32_t wz,
-                                                uint32_t colour, uint32_t sh, uint32_t faces)
-{
-    uint64_t r = (uint64_t)(uint16_t)wx | ((uint64_t)(uint16_t)wy << 16) |
-                 ((uint64_t)(uint16_t)wz << 32);
-    if constexpr (V2)
-        return r | ((uint64_t)(colour & 0xFFu) << 48) | ((uint64_t)(faces | (sh << 6)) << 56);
-    else
-        return r | ((uint64_t)(uint16_t)(colour | (sh << 6)) << 48);
-}
-
-template <int BS>
-__device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t *wsum, uint32_t &total)
-{
-    constexpr int NW = BS / 64;
-    const uint32_t lane = lane_id(), w = threadIdx.x >> 6;
-    uint32_t x = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        uint32_t y = __shfl_up(x, d, 64);
-        if (lane >= (uint32_t)d) x += y;
-    }
-    if (lane == 63) wsum[w] = x;
-    __syncthreads();
-    if (w == 0) {
-        uint32_t s = lane < (uint32_t)NW ? wsum[lane] : 0u, t = s;
-#pragma unroll
-        for (int d = 1; d < NW; d <<= 1) {
-            uint32_t y = __shfl_up(t, d, 64);
-            if (lane >= (uint32_t)d) t += y;
-        }
-        if (lane < (uint32_t)NW) wsum[lane] = t - s;      // exclusive wave base
-        if (lane == (uint32_t)NW - 1) wsum[NW] = t;       // block total
-    }
-    __syncthreads();
-    total = uni(wsum[NW]);
-    return wsum[w] + x - v;
-}
-
 // ---- emission ----------------------------------------------------------------
-// Exclusive prefix sum over the lanes of a wave, and the wave's total.
+// v of another lane by a DPP control word (0 where there is none).
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ uint32_t dpp0(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, true);
+}
+
+// Exclusive prefix sum over the lanes of a wave, and the wave's total: six
+// DPP additions (row_shr 1, 2, 4, 8, then the rows' totals), no LDS permutes.
 __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, uint32_t &total)
 {
-    const uint32_t ln = lane_id();
     uint32_t x = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_up((int)x, d, 64);
-        if (ln >= (uint32_t)d) x += y;
-    }
-    total = uni((uint32_t)__shfl((int)x, 63, 64));
+    x += dpp0<0x111>(x);
+    x += dpp0<0x112>(x);
+    x += dpp0<0x114>(x);
+    x += dpp0<0x118>(x);
+    x += dpp0<0x142, 0xA>(x);
+    x += dpp0<0x143, 0xC>(x);
+    total = (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
     return x - v;
 }
 
@@ -662,11 +613,17 @@ __device__ __forceinline__ void col1_row(const ChunkRefs &c, const uint64_t *lds
 // writes its row's cells (y << 7 | x) to the wave's list, and then the wave
 // writes the list's records with consecutive lanes on consecutive records,
 // U records per lane in flight.  A slice with more than LCAP cells goes in
-// batches of whole rows.  Colours are byte loads from the chunk (or from the
-// neighbour planes for cells at coordinate R); the shadow bits read a window
-// of the one map row the slice samples, staged in the wave's LDS area.
+// batches of whole rows; the cells of row y = R of a level-0 slice follow.
+//
+// The record loop is bound by its instructions, so everything that is the same
+// for a slice is prepared outside it: the shadow window holds, per map entry
+// pair, the height up to which the pair shadows (relative to the chunk, one
+// byte), so a cell compares once; a slice's voxels are a 4 KiB descriptor
+// (empty for a uniform chunk, whose value is the fill), so a colour is one load
+// at y R + x; and the records of a batch are a descriptor, so the lanes past
+// the batch need no branch.
 template <int B, int BS, bool V2, int U>
-__device__ void emit_slices(const CullArgs &a, const ChunkRefs &c, uint64_t *lds, uint64_t *out)
+__device__ __forceinline__ void emit_slices(const CullArgs &a, const ChunkRefs &c, uint64_t *lds, uint64_t *out)
 {
     using L = Lay<B, BS, V2>;
     using G = Geo<B>;
@@ -677,14 +634,14 @@ __device__ void emit_slices(const CullArgs &a, const ChunkRefs &c, uint64_t *lds
     using LE = typename std::conditional<L::MIP, uint16_t, uint32_t>::type;
     const uint8_t *xc = reinterpret_cast<const uint8_t *>(lds + L::XCB);
     LE *list = reinterpret_cast<LE *>(lds + L::WAVES + (int)w * L::WAVE_WORDS);
-    uint16_t *win = reinterpret_cast<uint16_t *>(list + LCAP);
+    uint8_t *win = reinterpret_cast<uint8_t *>(list + LCAP);
     const int nitems = a.lod ? L::NSLICES : L::SLB1;
     auto take = [&]() -> uint32_t {
         uint32_t t = 0;
         if (ln == 0)
             t = __hip_atomic_fetch_add(&soff[L::ITEM_U32], 1u, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_WORKGROUP);
-        return uni((uint32_t)__shfl((int)t, 0, 64));
+        return uni(t);
     };
     auto level_of = [](uint32_t t) {
         return (int)t < L::SLB1 ? 0 : (int)t < L::SLB2 ? 1 : (int)t < L::SLB3 ? 2
@@ -694,7 +651,7 @@ __device__ void emit_slices(const CullArgs &a, const ChunkRefs &c, uint64_t *lds
         return (int)t - (lv == 0 ? L::SLB0 : lv == 1 ? L::SLB1 : lv == 2 ? L::SLB2
                         : lv == 3 ? L::SLB3 : L::SLB4);
     };
-    // The shadow-map row a slice samples (2R + 2 entries, lane e holds e,
+    // The shadow-map row a slice samples (2R + 2 entries; lane e holds pairs e,
     // e + 64, e + 128) is loaded into registers one item ahead, so its wait
     // overlaps the previous slice's work.
     constexpr int WQ = (SWIN + 63) / 64;
@@ -708,7 +665,28 @@ __device__ void emit_slices(const CullArgs &a, const ChunkRefs &c, uint64_t *lds
                           c.org[0] + c.org[1] + 2u * dd;
 #pragma unroll
         for (int q = 0; q < WQ; q++)
-            if ((int)ln + 64 * q < SWIN) wv[q] = a.map[wb + ln + 64 * q];
+            if ((int)ln + 64 * q < SWIN) __builtin_memcpy(&wv[q], a.map + wb + ln + 64 * q, 4);
+    };
+    // a batch's records: U per lane in flight, make(entry, lo, hi) fills one
+    auto write = [&](uint64_t *ob, uint32_t nb, auto &&load, auto &&make) {
+        const __amdgpu_buffer_rsrc_t ro = byte_rsrc(ob, nb * 8u);
+        const uint32_t jmax = nb - 1u;
+#pragma unroll 1
+        for (uint32_t j0 = 0; j0 < nb; j0 += 64 * U) {
+            uint32_t e[U], col[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint32_t j = j0 + (uint32_t)u * 64u + ln;
+                e[u] = list[min(j, jmax)];
+                col[u] = load(e[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                uint32_t lo, hi;
+                make(e[u], col[u], lo, hi);
+                st8_nt(ro, (j0 + (uint32_t)u * 64u + ln) * 8u, lo, hi);
+            }
+        }
     };
     uint32_t nxt = take();
     uint32_t wv[WQ];
@@ -719,14 +697,16 @@ __device__ void emit_slices(const CullArgs &a, const ChunkRefs &c, uint64_t *lds
         if ((int)it >= nitems) break;
         const int l = level_of(it), s = slice_of(it, l);
         const int nl = G::n(l);
-        const uint32_t sbeg = soff[it], T = soff[it + 1] - sbeg;
+        const uint32_t sbeg = uni(soff[it]), T = uni(soff[it + 1]) - sbeg;
         const uint32_t d = l ? (1u << l) : 0u;        // LOD samples at +(1 << l) (mesher.c:523-531)
         if (T != 0) {
             wave_sync();                               // the previous slice's window reads are done
-            if (a.map) {
 #pragma unroll
-                for (int q = 0; q < WQ; q++)
-                    if ((int)ln + 64 * q < SWIN) win[ln + 64 * q] = (uint16_t)wv[q];
+            for (int q = 0; q < WQ; q++) {
+                // shadowed iff either entry is above wy = org + y (shadow.h:54-63)
+                const int h = (int)max(wv[q] & 0xFFFFu, wv[q] >> 16) - (int)c.org[1];
+                if ((int)ln + 64 * q < SWIN)
+                    win[ln + 64 * q] = (uint8_t)(a.map ? min(max(h, 0), 255) : 0);
             }
         }
         nxt = take();
@@ -734,138 +714,136 @@ __device__ void emit_slices(const CullArgs &a, const ChunkRefs &c, uint64_t *lds
         if (T == 0) continue;
         const uint64_t *rows = l == 0 ? lds + L::V0 + s * N0
                                       : lds + L::P1 + (G::row_base(l) - G::RB1) + s * nl;
+        const int lanes = l == 0 ? R : nl;             // row y = R of level 0 comes last
         uint64_t rb = 0;
         uint32_t xb = 0;
-        if ((int)ln < nl) rb = rows[ln];
+        if ((int)ln < lanes) rb = rows[ln];
         if (l == 0 && s < R && (int)ln < R) xb = (uint32_t)(lds[L::XB + s] >> ln) & 1u;
         const uint32_t cnt = (uint32_t)__popcll(rb) + xb;
-        uint32_t tot64;
-        const uint32_t off = wave_excl_scan(cnt, tot64);
-        const uint64_t rbx = nl > 64 ? rows[64] : 0ull;    // row y = 64 of level 0 (R = 64)
-        uint64_t pdz = 0, pdy = 0, pdx = 0;     // level-1 child planes of lane's row
+        uint32_t tot;
+        const uint32_t off = wave_excl_scan(cnt, tot);
         uint64_t *o = out + sbeg;
         const uint32_t wz = c.org[2] + ((uint32_t)s << l);
+        const uint32_t base = c.org[0] | c.org[1] << 16;   // + x + (y << 16): no carries
 #pragma unroll 1
-        for (uint32_t b0 = 0; b0 < T;) {
+        for (uint32_t b0 = 0; b0 < tot;) {
             const uint32_t lim = b0 + LCAP;
-            const bool pending = cnt && off >= b0;
-            uint32_t b1 = wave_min(pending && off + cnt > lim ? off : 0xFFFFFFFFu);
-            if (b1 == 0xFFFFFFFFu) b1 = T <= lim ? T : tot64;
+            uint32_t b1 = tot;
+            if (tot > lim) b1 = wave_min(cnt && off >= b0 && off + cnt > lim ? off : 0xFFFFFFFFu);
             wave_sync();                               // the previous batch's list reads are done
-            if (pending && off < b1) {
-                uint32_t pos = off - b0;
-                uint64_t m = rb;
+            if (cnt && off >= b0 && off < b1) {
+                LE *q = list + (off - b0);
                 const uint32_t code = ln << 7;
-                if (!L::MIP && l == 1) {
-                    // level 1: the descent to the level-0 child for the whole row
-                    // at once, as bit planes over X (the child's dz, dy, dx)
-                    l1_child_planes<B, V2>(lds, s, (int)ln, pdz, pdy, pdx);
+                // level 1 without the colour mip: the level-0 child each cell
+                // descends to, for the whole row at once, as bit planes over X
+                uint64_t pdz = 0, pdy = 0, pdx = 0;
+                const bool sel = !L::MIP && l == 1;
+                if (sel) l1_child_planes<B, V2>(lds, s, (int)ln, pdz, pdy, pdx);
+                auto half = [&](uint32_t m, uint32_t x0) {
                     while (m) {
-                        const uint32_t x = (uint32_t)__builtin_ctzll(m);
-                        m &= m - 1ull;
-                        const uint32_t sel = (uint32_t)((pdz >> x) & 1ull) |
-                                             ((uint32_t)((pdy >> x) & 1ull) << 1) |
-                                             ((uint32_t)((pdx >> x) & 1ull) << 2);
-                        list[pos++] = (LE)(code | x | (sel << 16));
+                        const uint32_t x = x0 + (uint32_t)__builtin_ctz(m);
+                        m &= m - 1u;
+                        uint32_t e = code | x;
+                        if (sel)
+                            e |= (uint32_t)((pdz >> x) & 1ull) << 16 |
+                                 (uint32_t)((pdy >> x) & 1ull) << 17 |
+                                 (uint32_t)((pdx >> x) & 1ull) << 18;
+                        *q++ = (LE)e;
                     }
-                } else {
-                    while (m) {
-                        const uint32_t x = (uint32_t)__builtin_ctzll(m);
-                        m &= m - 1ull;
-                        list[pos++] = (LE)(code | x);
-                    }
-                    if (xb) list[pos] = (LE)(code | (uint32_t)R);
-                }
+                };
+                half((uint32_t)rb, 0u);
+                half((uint32_t)(rb >> 32), 32u);
+                if (xb) *q = (LE)(code | (uint32_t)R);
             }
-            if (rbx && b1 == T && tot64 >= b0 && ((rbx >> ln) & 1ull))
-                list[tot64 - b0 + rank_below(rbx)] = (LE)((64u << 7) | ln);
             wave_sync();
             const uint32_t nb = b1 - b0;
-            uint64_t *ob = o + b0;
             if (l == 0) {
-                // The colour loads of a round go out together, with no branch
-                // around them: lanes past the end of the batch take its last
-                // entry and store that entry's record again, to the same
-                // place.  (With a branch per record the compiler waited for
-                // each load in turn: loads and stores share one completion
-                // counter here, so it cannot wait for a subset.)
-                const uint32_t jmax = nb - 1u;
-#pragma unroll 1
-                for (uint32_t j0 = 0; j0 < nb; j0 += 64 * U) {
-                    uint32_t col[U];
-                    uint64_t rec[U];
-#pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        const uint32_t j = j0 + (uint32_t)u * 64u + ln;
-                        const uint32_t e = list[j < jmax ? j : jmax];
-                        const int x = (int)(e & 127u), y = (int)((e >> 7) & 127u);
-                        col[u] = cell_colour<B>(c, xc, x, y, s);
-                        const uint32_t wy = c.org[1] + (uint32_t)y;
-                        uint32_t sh = 0;
-                        if (a.map) sh = !(win[x + y] <= wy && win[x + y + 1] <= wy);
-                        uint32_t fl = 0;
-                        if constexpr (V2) fl = face_flags<B, V2>(lds, x, y, s);
-                        rec[u] = pack_record<V2>(c.org[0] + (uint32_t)x, wy, wz, 0u, sh, fl);
-                    }
-#pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        const uint32_t j = j0 + (uint32_t)u * 64u + ln;
-                        __builtin_nontemporal_store(rec[u] | ((uint64_t)(col[u] & 0xFFu) << 48),
-                                                    &ob[j < jmax ? j : jmax]);
-                    }
-                }
+                const int u = s < R ? c.own_u : c.nb_u[2];
+                const uint8_t *p = s < R ? c.own + (size_t)s * R * R : c.nb[2];
+                const __amdgpu_buffer_rsrc_t rc = byte_rsrc(p, u < 0 ? (uint32_t)(R * R) : 0u);
+                const uint32_t fill = u < 0 ? 0u : (uint32_t)u;
+                const uint8_t *xs = xc + s * R;
+                write(o + b0, nb,
+                      [&](uint32_t e) {
+                          return (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(
+                              rc, (int)(((e >> 7) << B) + (e & 127u)), 0, 0);
+                      },
+                      [&](uint32_t e, uint32_t col, uint32_t &lo, uint32_t &hi) {
+                          const uint32_t x = e & 127u, y = e >> 7;
+                          col |= fill;
+                          if (x == (uint32_t)R) col = xs[y];
+                          const bool sh = win[x + y] > y;
+                          lo = base + x + (y << 16);
+                          if constexpr (V2)
+                              hi = wz | col << 16 |
+                                   face_flags<B, V2>(lds, (int)x, (int)y, s) << 24 |
+                                   (sh ? 1u << 30 : 0u);
+                          else
+                              hi = (col << 16 | (sh ? 1u << 22 : 0u)) | wz;
+                      });
+            } else if constexpr (L::MIP) {
+                const uint8_t *colm = reinterpret_cast<const uint8_t *>(lds + L::COL) +
+                                      L::cbase(l) + s * nl * nl;
+                write(o + b0, nb,
+                      [&](uint32_t e) {
+                          return (uint32_t)colm[__umul24(e >> 7, (uint32_t)nl) + (e & 127u)];
+                      },
+                      [&](uint32_t e, uint32_t col, uint32_t &lo, uint32_t &hi) {
+                          const uint32_t x = (e & 127u) << l, y = (e >> 7) << l;
+                          const bool sh = win[x + y] > y + d;
+                          lo = base + x + (y << 16);
+                          hi = (col << 16 | (sh ? 1u << 22 : 0u)) | wz;
+                      });
             } else {
-                const uint8_t *colm = reinterpret_cast<const uint8_t *>(lds + L::COL) + L::cbase(l);
-#pragma unroll 1
-                for (uint32_t j0 = 0; j0 < nb; j0 += 64 * U) {
-                    uint32_t col[U];
-                    uint64_t rec[U];
-#pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        const uint32_t j = j0 + (uint32_t)u * 64u + ln;
-                        col[u] = 0;
-                        rec[u] = 0;
-                        if (j < nb) {
-                            const uint32_t e = list[j];
-                            const int X = (int)(e & 127u), Y = (int)((e >> 7) & 127u);
-                            int qx = X, qy = Y, qz = s;
-                            if constexpr (L::MIP) {
-                                col[u] = colm[(s * nl + Y) * nl + X];
-                            } else {
-                                if (l == 1) {
-                                    qz = 2 * s + (int)((e >> 16) & 1u);
-                                    qy = 2 * Y + (int)((e >> 17) & 1u);
-                                    qx = 2 * X + (int)((e >> 18) & 1u);
-                                } else {
-                                    descend_bf<B, V2>(lds, l, qx, qy, qz);
-                                }
-                                col[u] = cell_colour<B>(c, xc, qx, qy, qz);
-                            }
-                            const uint32_t wy = c.org[1] + ((uint32_t)Y << l);
-                            const uint32_t ex = (uint32_t)(X + Y) << l;
-                            uint32_t sh = 0;
-                            if (a.map) sh = !(win[ex] <= wy + d && win[ex + 1] <= wy + d);
-                            uint32_t fl = 0;
-                            if constexpr (V2) fl = face_flags<B, V2>(lds, qx, qy, qz);
-                            rec[u] = pack_record<V2>(c.org[0] + ((uint32_t)X << l), wy, wz, 0u,
-                                                     sh, fl);
-                        }
+                // the level-0 cell an entry's colour (and faces) come from
+                auto child = [&](uint32_t e, int &qx, int &qy, int &qz) {
+                    qx = (int)(e & 127u);
+                    qy = (int)((e >> 7) & 127u);
+                    qz = s;
+                    if (l == 1) {
+                        qz = 2 * qz + (int)((e >> 16) & 1u);
+                        qy = 2 * qy + (int)((e >> 17) & 1u);
+                        qx = 2 * qx + (int)((e >> 18) & 1u);
+                    } else {
+                        descend_bf<B, V2>(lds, l, qx, qy, qz);
                     }
-#pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        const uint32_t j = j0 + (uint32_t)u * 64u + ln;
-                        if (j < nb) __builtin_nontemporal_store(rec[u] | ((uint64_t)(col[u] & 0xFFu) << 48), &ob[j]);
-                    }
-                }
+                };
+                write(o + b0, nb,
+                      [&](uint32_t e) {
+                          int qx, qy, qz;
+                          child(e, qx, qy, qz);
+                          uint32_t f = 0;
+                          if constexpr (V2) f = face_flags<B, V2>(lds, qx, qy, qz);
+                          return cell_colour<B>(c, xc, qx, qy, qz) | f << 8;
+                      },
+                      [&](uint32_t e, uint32_t col, uint32_t &lo, uint32_t &hi) {
+                          const uint32_t x = (e & 127u) << l, y = ((e >> 7) & 127u) << l;
+                          const bool sh = win[x + y] > y + d;
+                          lo = base + x + (y << 16);
+                          hi = (col << 16 | (sh ? (V2 ? 1u << 30 : 1u << 22) : 0u)) | wz;
+                      });
             }
             b0 = b1;
+        }
+        if (l == 0 && tot < T) {
+            // row y = R: cells of the +y neighbour, lane x holds cell x
+            const uint64_t rx = uni(rows[R]);
+            if ((rx >> ln) & 1ull) {
+                const uint32_t col = c.nb_u[1] >= 0 ? (uint32_t)c.nb_u[1]
+                                                    : (uint32_t)c.nb[1][(size_t)s * R * R + ln];
+                const bool sh = win[ln + R] > R;
+                const uint32_t lo = base + ln + ((uint32_t)R << 16);
+                const uint32_t hi = wz | col << 16 |
+                                    (V2 ? 8u << 24 | (sh ? 1u << 30 : 0u) : (sh ? 1u << 22 : 0u));
+                __builtin_nontemporal_store((uint64_t)hi << 32 | lo, o + tot + rank_below(rx));
+            }
         }
     }
 }
 
 // Work for one chunk; all threads of the workgroup call it.
 template <int B, int BS, bool V2, bool MASK_OUT, int U>
-__device__ void cull_chunk(const CullArgs &a, uint32_t k, uint32_t n, uint64_t *lds,
+__device__ __forceinline__ void cull_chunk(const CullArgs &a, uint32_t k, uint32_t n, uint64_t *lds,
                            uint32_t *wsum, uint64_t *s_base)
 {
     using G = Geo<B>;

@@ -623,7 +623,8 @@ __device__ __forceinline__ void col1_row(const ChunkRefs &c, const uint64_t *lds
 // at y R + x; and the records of a batch are a descriptor, so the lanes past
 // the batch need no branch.
 template <int B, int BS, bool V2, int U>
-__device__ __forceinline__ void emit_slices(const CullArgs &a, const ChunkRefs &c, uint64_t *lds, uint64_t *out)
+__device__ __forceinline__ void emit_slices(const CullArgs &a, const ChunkRefs &c, uint64_t *lds, uint64_t *out,
+                                            uint32_t part, uint32_t parts)
 {
     using L = Lay<B, BS, V2>;
     using G = Geo<B>;
@@ -641,7 +642,7 @@ __device__ __forceinline__ void emit_slices(const CullArgs &a, const ChunkRefs &
         if (ln == 0)
             t = __hip_atomic_fetch_add(&soff[L::ITEM_U32], 1u, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_WORKGROUP);
-        return uni(t);
+        return uni(t) * parts + part;
     };
     auto level_of = [](uint32_t t) {
         return (int)t < L::SLB1 ? 0 : (int)t < L::SLB2 ? 1 : (int)t < L::SLB3 ? 2
@@ -841,10 +842,12 @@ __device__ __forceinline__ void emit_slices(const CullArgs &a, const ChunkRefs &
     }
 }
 
-// Work for one chunk; all threads of the workgroup call it.
+// Work for part `part` of `parts` of one chunk; all threads of the workgroup
+// call it.  Every part culls and counts the whole chunk; the first one
+// publishes its sizes, and part p emits the z-slices p, p + parts, ...
 template <int B, int BS, bool V2, bool MASK_OUT, int U>
 __device__ __forceinline__ void cull_chunk(const CullArgs &a, uint32_t k, uint32_t n, uint64_t *lds,
-                           uint32_t *wsum, uint64_t *s_base)
+                           uint32_t *wsum, uint64_t *s_base, uint32_t part = 0, uint32_t parts = 1)
 {
     using G = Geo<B>;
     using L = Lay<B, BS, V2>;
@@ -1138,9 +1141,9 @@ __device__ __forceinline__ void cull_chunk(const CullArgs &a, uint32_t k, uint32
         uint64_t excl = 0;
         if (!a.single) {
             if (k == 0) {
-                if (threadIdx.x == 0) st_relaxed(a.state, kFlagPre | items);
+                if (threadIdx.x == 0 && part == 0) st_relaxed(a.state, kFlagPre | items);
             } else {
-                if (threadIdx.x == 0) st_relaxed(a.state + k, kFlagAgg | items);
+                if (threadIdx.x == 0 && part == 0) st_relaxed(a.state + k, kFlagAgg | items);
                 int64_t top = (int64_t)k - 1;       // nearest predecessor not yet summed
                 const uint32_t ln = lane_id();
                 for (;;) {
@@ -1162,11 +1165,12 @@ __device__ __forceinline__ void cull_chunk(const CullArgs &a, uint32_t k, uint32
                     if (pre) break;
                     top -= 64;
                 }
-                if (threadIdx.x == 0) st_relaxed(a.state + k, kFlagPre | (excl + items));
+                if (threadIdx.x == 0 && part == 0)
+                    st_relaxed(a.state + k, kFlagPre | (excl + items));
             }
         }
-        if (threadIdx.x == 0) {
-            *s_base = excl;
+        if (threadIdx.x == 0) *s_base = excl;
+        if (threadIdx.x == 0 && part == 0) {
             a.offsets[k] = excl;
             if (k + 1 == n) a.offsets[n] = excl + items;
             for (int l = 0; l < 5; l++) a.level_counts[(size_t)k * 5 + l] = 4u * lvl[l];
@@ -1180,7 +1184,21 @@ __device__ __forceinline__ void cull_chunk(const CullArgs &a, uint32_t k, uint32
     if (base + total > a.cap) return;
 
     // ---- 5. emission: waves take z-slices from the work counter ----
-    emit_slices<B, BS, V2, U>(a, c, lds, a.splats + base);
+    emit_slices<B, BS, V2, U>(a, c, lds, a.splats + base, part, parts);
+}
+
+// A list too short to fill the chip hands each chunk to several workgroups.
+// A 64^3 chunk's workgroup spends most of its time on the emission, whose
+// z-slices are independent ranges of the output, so the parts repeat the cull
+// and count (reads that the caches serve) and share the slices out: one 64^3
+// chunk 47.3 -> 28.9 us, the 32 chunks of a few edits 178 -> 45-48 us.  At most
+// R / 4 of them: the slices left to a part then cost less than its cull.
+template <int B>
+constexpr uint32_t max_parts() { return B < 2 ? 1u : 1u << (B - 2); }
+
+static uint32_t max_parts_of(uint32_t root_bitw, bool count_only)
+{
+    return count_only || root_bitw < 2 ? 1u : 1u << (root_bitw - 2);
 }
 
 // LDS (about 67 KiB at 512 threads for R = 64) allows two workgroups per CU;
@@ -1195,8 +1213,8 @@ __attribute__((amdgpu_waves_per_eu(BS == 256 ? 2 : 4))) k_cull(CullArgs a)
     __shared__ uint32_t wsum[BS / 64 + 1];
     __shared__ uint32_t s_ticket;
     __shared__ uint64_t s_base;
-    if (a.single) {
-        cull_chunk<B, BS, V2, MASK_OUT, U>(a, 0u, 1u, lds, wsum, &s_base);
+    if (a.single) {       // one workgroup per part
+        cull_chunk<B, BS, V2, MASK_OUT, U>(a, 0u, 1u, lds, wsum, &s_base, blockIdx.x, gridDim.x);
         return;
     }
     if (MASK_OUT) {   // make_mask: one workgroup per listed chunk, no offsets
@@ -1207,12 +1225,18 @@ __attribute__((amdgpu_waves_per_eu(BS == 256 ? 2 : 4))) k_cull(CullArgs a)
         return;
     }
     const uint32_t n = a.d_n ? min(*a.d_n, a.n) : a.n;
+    // whole multiples of the list that the grid holds at once: more parts than
+    // workgroups would put a second round of culls behind the first.  Tickets
+    // run chunk by chunk, so the parts a look-back waits for have lower ones.
+    const uint32_t parts = a.count_only || n == 0u
+                               ? 1u : max(1u, min(max_parts<B>(), gridDim.x / n));
     for (;;) {
         if (threadIdx.x == 0) s_ticket = atomicAdd(a.ticket, 1u);
         __syncthreads();
-        const uint32_t k = uni(s_ticket);
+        const uint32_t t = uni(s_ticket);
+        const uint32_t k = parts > 1u ? t / parts : t;
         if (k >= n) break;
-        cull_chunk<B, BS, V2, MASK_OUT, U>(a, k, n, lds, wsum, &s_base);
+        cull_chunk<B, BS, V2, MASK_OUT, U>(a, k, n, lds, wsum, &s_base, t - k * parts, parts);
         __syncthreads();
     }
 }
@@ -1339,7 +1363,8 @@ int cull_mesh_launch(vp_ctx *ctx, const vp_world_desc *world, const uint8_t *d_v
     a.status = ctx->d_status;
     a.nchunks = (uint32_t)(1ull << (world->max_bitw[0] + world->max_bitw[1] + world->max_bitw[2]));
     const vp_remesh_shape_i sh = remesh_shape(ctx, world);
-    int grid = 1, bs = sh.block;
+    const uint32_t parts = max_parts_of(world->root_bitw, a.count_only != 0);
+    int grid = a.single ? (int)parts : 1, bs = sh.block;
     // one 64^3 chunk alone: a 1024-thread workgroup (16 waves on one CU)
     // finishes it in 0.70x the time of the batched path's 512-thread shape
     if (a.single && world->root_bitw == 6) bs = 1024;
@@ -1348,7 +1373,7 @@ int cull_mesh_launch(vp_ctx *ctx, const vp_world_desc *world, const uint8_t *d_v
         a.ticket = ticket;
         a.state = state;
         const int resident = ctx->num_cus * sh.wg_per_cu;
-        grid = (int)((uint64_t)n < (uint64_t)resident ? n : (uint32_t)resident);
+        grid = (int)((uint64_t)n * parts < (uint64_t)resident ? n * parts : (uint32_t)resident);
         const int rgrid = (int)((n + 255u) / 256u);
         hipLaunchKernelGGL(k_cull_reset, dim3(rgrid < 1024 ? rgrid : 1024), dim3(256), 0, st,
                            a.ticket, a.state, n, a.offsets);

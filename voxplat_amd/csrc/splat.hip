@@ -755,6 +755,18 @@ __device__ __forceinline__ bool splat_open(const uint2 rec, float lodf, const Sp
     return far >= lb;
 }
 
+// Blocks whose splats are at least this many pixels wide are handed out in
+// quarters: their sprites cost so much that a wave with a whole block of them
+// outlasts the others (15 views of 425x425 close to a 7.9 M list: 2954 against
+// 3332 us; 2422x2321: 1010 against 1190 us).  Farther blocks are cheaper whole,
+// one look at their bounds each (all of them in quarters: 1.2x the time).
+constexpr float kNearPixels = 5.0f;
+// Frames of up to this many pixels are rasterised without the tile bounds: the
+// whole frame stays in the L2s, and rejecting a fragment by its own load is
+// then cheaper than a pass over bounds (183x151 of a 65 M list: 340 against
+// 421 us, 489x499 of 114 M: 524 against 552 us; 757x591: 489 against 498 us, and
+// 928x743 of 3.3 M: 152 against 131 us).
+constexpr uint64_t kFewPixels = 1u << 18;
 constexpr uint32_t kHeld = kBlock + 64;   // a wave's queue: less than a wave, and a block
 // Wave w takes the ordered blocks w, w + G, w + 2G, ... (G waves): every wave
 // starts at the near end of the order, no counter is shared, and the waves
@@ -777,7 +789,8 @@ __global__ void __launch_bounds__(kBlock) k_raster_blocks(const int16_t *splats,
                                                            const uint4 *box, uint32_t *hiz,
                                                            const uint32_t *cnt,
                                                            const uint64_t *d_n,
-                                                           const uint32_t *tiles_ok)
+                                                           const uint32_t *tiles_ok,
+                                                           uint32_t near_bin)
 {
     // splats that may still win a pixel: record, index and level
     struct Held {
@@ -803,14 +816,19 @@ __global__ void __launch_bounds__(kBlock) k_raster_blocks(const int16_t *splats,
         const uint2 rec = ok ? make_uint2(q.x[e], q.y[e]) : make_uint2(0u, 0u);
         raster_splat(ok, rec, ok ? (float)(1u << q.lv[e]) : 1.0f, ok ? q.id[e] : 0u, c, rays, frame);
     };
+    // units of work: the quarters of the near blocks (those of the first near_bin
+    // bins, whose cursors ended at the bins' ends), then whole blocks
+    const uint32_t near = near_bin ? cnt[kBins + near_bin - 1u] : 0u, units = total + 3u * near;
     // one block ahead: its box and its first tile bounds, so that their loads
     // are in flight while the block before it is worked on
-    uint32_t b = 0, lb = 0, first = 0;
+    uint32_t b = 0, lb = 0, first = 0, part = 0;
     BoxWalk walk = {};
     uint2 rec[PER];
     uint32_t lv[PER];
     auto fetch = [&](uint32_t t) {
-        b = (uint32_t)__builtin_amdgcn_readfirstlane((int)order[t]);
+        const bool quarter = t < 4u * near;
+        b = (uint32_t)__builtin_amdgcn_readfirstlane((int)order[quarter ? t >> 2 : t - 3u * near]);
+        part = quarter ? 1u << (t & 3u) : (1u << PER) - 1u;
         const uint4 bx = box[b];
         lb = bx.z;
         walk = box_walk(bx);
@@ -822,14 +840,15 @@ __global__ void __launch_bounds__(kBlock) k_raster_blocks(const int16_t *splats,
             const uint64_t i = (uint64_t)b * kBlock + (uint64_t)(k * 64) + lane;
             rec[k] = make_uint2(0u, 0u);
             lv[k] = lod_log2;
+            if (!((part >> k) & 1u)) continue;
             if (i < n) {
                 rec[k] = *reinterpret_cast<const uint2 *>(splats + 4 * i);
                 if (lod) lv[k] = lod[i];
             }
         }
     };
-    if (w < total) fetch(w);
-    for (uint32_t t = w; t < total; t += nw) {
+    if (w < units) fetch(w);
+    for (uint32_t t = w; t < units; t += nw) {
         const bool hidden = box_hidden(walk, lb, first, hiz, tx);
         if (!hidden) {
             records();
@@ -837,10 +856,12 @@ __global__ void __launch_bounds__(kBlock) k_raster_blocks(const int16_t *splats,
 #pragma unroll
             for (int k = 0; k < PER; k++) {
                 const uint64_t i = (uint64_t)b * kBlock + (uint64_t)(k * 64) + lane;
-                open[k] = i < n && splat_open(rec[k], (float)(1u << lv[k]), c, hiz, tx);
+                open[k] = ((part >> k) & 1u) && i < n &&
+                          splat_open(rec[k], (float)(1u << lv[k]), c, hiz, tx);
             }
 #pragma unroll
             for (int k = 0; k < PER; k++) {
+                if (!((part >> k) & 1u)) continue;
                 const uint64_t m = __ballot(open[k]);
                 const uint32_t e = held + __builtin_amdgcn_mbcnt_hi(
                     (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
@@ -853,7 +874,7 @@ __global__ void __launch_bounds__(kBlock) k_raster_blocks(const int16_t *splats,
                 held += (uint32_t)__popcll(m);
             }
         }
-        if (t + nw < total) fetch(t + nw);
+        if (t + nw < units) fetch(t + nw);
         wave_fence();
         while (held >= 64) {
             held -= 64;
@@ -863,6 +884,30 @@ __global__ void __launch_bounds__(kBlock) k_raster_blocks(const int16_t *splats,
         if (++turn & 1u) hiz_refresh(frame, hiz, c.W, c.H, h0, h1);
     }
     flush(0u, lane < held);
+}
+
+// The visible blocks without the tile bounds (frames of up to kFewPixels): a
+// workgroup per block, a splat per thread.
+__global__ void __launch_bounds__(kBlock) k_raster_few(const int16_t *splats, const uint8_t *lod,
+                                                        uint32_t lod_log2, uint64_t n, SplatCam c,
+                                                        const float4 *rays, uint64_t *frame,
+                                                        const uint32_t *order,
+                                                        const uint32_t *cnt, const uint64_t *d_n,
+                                                        const uint32_t *tiles_ok)
+{
+    if (tiles_ok && *tiles_ok) return;    // the screen-tile path resolved this frame
+    const uint32_t total = cnt[kTotal];
+    if (d_n) n = min(*d_n, n);
+    for (uint32_t t = blockIdx.x; t < total; t += gridDim.x) {
+        const uint64_t i = (uint64_t)order[t] * kBlock + threadIdx.x;
+        uint2 rec = make_uint2(0u, 0u);
+        uint32_t lv = lod_log2;
+        if (i < n) {
+            rec = *reinterpret_cast<const uint2 *>(splats + 4 * i);
+            if (lod) lv = lod[i];
+        }
+        raster_splat(i < n, rec, (float)(1u << lv), (uint32_t)i, c, rays, frame);
+    }
 }
 
 // ---- screen-tile resolve ------------------------------------------------------
@@ -1469,9 +1514,20 @@ static int splat_frame(vp_ctx *ctx, const int16_t *d_splats, const uint8_t *d_lo
         // 4 workgroups per CU: fewer hide less latency (3: 1248 us against
         // 1090 for the 1080p frame), more start further from the near end
         // before anything is hidden (6 resident: 911 against 879 us)
-        hipLaunchKernelGGL(k_raster_blocks, dim3((uint32_t)ncu * 4u), dim3(kBlock), 0, st,
-                           d_splats, d_lod, lod_log2, n, c, rays, frame, order, box, hiz, cnt, d_n,
-                           tiles ? tb.tc + kTcOk : nullptr);
+        const dim3 grid((uint32_t)ncu * 4u);
+        const uint32_t *ok = tiles ? tb.tc + kTcOk : nullptr;
+        if (np <= kFewPixels) {
+            hipLaunchKernelGGL(k_raster_few, grid, dim3(kBlock), 0, st, d_splats, d_lod, lod_log2,
+                               n, c, rays, frame, order, cnt, d_n, ok);
+        } else {
+            // the distance at which a splat is kNearPixels wide, as block_bin's bin
+            const float reach = (float)c.H * 1.1f * (float)(1u << lod_log2) / kNearPixels;
+            const float bin = sqrtf(reach / c.far_plane) * (float)kBins;
+            const uint32_t near_bin = (uint32_t)fminf(fmaxf(bin, 0.0f), (float)kBins);
+            hipLaunchKernelGGL(k_raster_blocks, grid, dim3(kBlock), 0, st, d_splats, d_lod,
+                               lod_log2, n, c, rays, frame, order, box, hiz, cnt, d_n, ok,
+                               near_bin);
+        }
     } else if (n) {
         hipLaunchKernelGGL(k_raster, dim3((uint32_t)nb), dim3(256), 0, st, d_splats, d_lod,
                            lod_log2, n, c, rays, frame);

@@ -398,28 +398,6 @@ __device__ __forceinline__ uint32_t face_flags(const uint64_t *lds, int x, int y
 }
 
 // ---- emission ----------------------------------------------------------------
-// v of another lane by a DPP control word (0 where there is none).
-template <int CTRL, int ROWS = 0xF>
-__device__ __forceinline__ uint32_t dpp0(uint32_t v)
-{
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, true);
-}
-
-// Exclusive prefix sum over the lanes of a wave, and the wave's total: six
-// DPP additions (row_shr 1, 2, 4, 8, then the rows' totals), no LDS permutes.
-__device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, uint32_t &total)
-{
-    uint32_t x = v;
-    x += dpp0<0x111>(x);
-    x += dpp0<0x112>(x);
-    x += dpp0<0x114>(x);
-    x += dpp0<0x118>(x);
-    x += dpp0<0x142, 0xA>(x);
-    x += dpp0<0x143, 0xC>(x);
-    total = (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
-    return x - v;
-}
-
 __device__ __forceinline__ uint32_t wave_min(uint32_t v)
 {
 #pragma unroll

@@ -14,11 +14,13 @@
 //  3. the chunk's word count is published and its output offset taken by a
 //     decoupled look-back (same scheme as the remesh kernel).
 //  4. each thread writes the words of its bitmap words.
-// Decode, one workgroup per chunk: a stream of one full-chunk run is a fill;
-// otherwise the words are read eight per thread at a time, their values kept
-// in LDS and their lengths scanned into start positions, set as bits of an
-// LDS bitmap; an output byte's run is the rank of the last start at or before
-// it, so every 16-byte store is independent.
+// Decode, one workgroup per chunk (or, of few chunks, several): a stream of one
+// full-chunk run is a fill; otherwise the words are read eight per thread at a
+// time, their values kept in LDS and their lengths scanned into start
+// positions, set as bits of an LDS bitmap; an output byte's run is the rank of
+// the last start at or before it, so every 16-byte store is independent.
+// Bound by its stores and by the scan's latency: a 2048x256x2048 world (1.07 GB
+// of voxels from 0.2 GB of words) 547 -> 268 us, 4.8 TB/s.
 #include "vp_internal.h"
 
 namespace vp {
@@ -42,6 +44,7 @@ struct RleArgs {
     uint32_t       *status;
     uint8_t         single;
     uint32_t        nchunks;
+    uint32_t        parts;         // workgroups that share a chunk's bytes (decode)
 };
 
 __device__ __forceinline__ uint32_t r_lane() { return threadIdx.x & 63u; }
@@ -309,22 +312,46 @@ __global__ void __launch_bounds__(BS) k_rle_encode(RleArgs a)
     }
 }
 
+// 16 bytes of stream words at any word address
+struct __attribute__((packed, aligned(4))) Words4 {
+    uint32_t w[4];
+};
+
 template <int B, int BS>
 __global__ void __launch_bounds__(BS) k_rle_decode(RleArgs a)
 {
     constexpr int R = 1 << B, VOX = R * R * R, WORDS = VOX / 64, WPT = (WORDS + BS - 1) / BS;
+    constexpr int NW = BS / 64;
     constexpr int K = 8;             // stream words per thread per batch, loads in flight
     // run values kept in LDS for streams of up to VCAP runs: at R = 64 what
-    // leaves two workgroups per CU (2 x 81.8 KB); a chunk with 5% of its
+    // leaves two workgroups per CU (2 x 81.9 KB); a chunk with 5% of its
     // voxels as single-voxel holes has about 26,000 runs
-    constexpr int VCAP = VOX < 32640 ? VOX : 32640;
+    constexpr int VCAP = VOX < 32448 ? VOX : 32448;
     constexpr uint32_t LMAX = (uint32_t)VOX + 1u;   // longer runs are malformed; clamped
     __shared__ uint64_t bm[WORDS];
     __shared__ uint32_t rank[WORDS];
-    __shared__ uint8_t val8[VCAP];
-    __shared__ uint32_t wsum[BS / 64 + 1];
+    __shared__ uint32_t val32[VCAP / 4 + 4];        // the value of run i is byte i + 1
+    __shared__ uint32_t wtot[WPT * NW > 2 * NW ? WPT * NW : 2 * NW];   // totals of the waves
     __shared__ uint32_t s_bad, s_nz;
-    for (uint32_t k = blockIdx.x; k < a.n; k += gridDim.x) {
+    static_assert(WPT * NW <= 64, "one wave scans the wave totals");
+    uint8_t *val8 = reinterpret_cast<uint8_t *>(val32);
+    uint32_t *bm32 = reinterpret_cast<uint32_t *>(bm);
+    const uint32_t ln = r_lane();
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    bool fresh = true;               // bm was never cleared; later each chunk leaves it clear
+    // Round r hands entries r G .. r G + G - 1 to the G workgroups, rotated by a
+    // golden-section step per round: with the plain stride a workgroup of a
+    // whole world meets the same height every time, all air or all caves.
+    // (2048x256x2048 world: 324 -> 265 us.)
+    const uint32_t G = gridDim.x / a.parts, turn = (uint32_t)(0.618f * (float)G) | 1u;
+    uint32_t slot = blockIdx.x / a.parts;
+    // a part's share of the chunk's 16-byte pieces, in multiples of the workgroup
+    const uint32_t part = blockIdx.x - slot * a.parts;
+    const int p_lo = (int)((uint32_t)(VOX / 16) / a.parts * part),
+              p_hi = p_lo + (int)((uint32_t)(VOX / 16) / a.parts);
+    for (uint64_t k0 = 0; k0 < a.n; k0 += G, slot = (slot + turn) % G) {
+        if (k0 + slot >= a.n) break;
+        const uint32_t k = (uint32_t)k0 + slot;
         const uint32_t chunk = a.ids[k];
         const uint64_t o0 = a.offsets[k], o1 = a.offsets[k + 1];
         if (chunk >= a.nchunks || o0 > o1 || o1 > a.cap) {
@@ -341,91 +368,179 @@ __global__ void __launch_bounds__(BS) k_rle_decode(RleArgs a)
                 const uint32_t b = w0 >> 24;
                 const uint32_t v4 = b * 0x01010101u;
                 const uint4 q = make_uint4(v4, v4, v4, v4);
-                for (int s = threadIdx.x; s < VOX / 16; s += BS)
+                for (int s = p_lo + (int)threadIdx.x; s < p_hi; s += BS)
                     nt_store16(dst + (size_t)s * 16, q);
                 continue;   // uniform across the workgroup
             }
         }
-        for (int w = threadIdx.x; w < WORDS; w += BS) bm[w] = 0ull;
-        // the runs end at the first 0 word after word 0 (rle.c:100-108: the
-        // first word is always expanded)
+        if (fresh)
+            for (int w = threadIdx.x; w < WORDS; w += BS) bm[w] = 0ull;
+        fresh = false;
+        // The runs end at the first 0 word after word 0 (rle.c:100-108: the
+        // first word is always expanded): the last word of a well-formed
+        // stream.  One found earlier takes its batch again.
+        uint64_t nz = avail;
+        if (avail >= 2 && wd[avail - 1] == 0u) nz = avail - 1;
         if (threadIdx.x == 0) {
             s_bad = 0u;
-            s_nz = (uint32_t)(avail < 0xFFFFFFFFull ? avail : 0xFFFFFFFFull);
+            s_nz = (uint32_t)(nz < 0xFFFFFFFFull ? nz : 0xFFFFFFFFull);
         }
         __syncthreads();
-        uint64_t nz = s_nz;
         // run starts: batches of K words per thread; the terminator search,
-        // the run values (into LDS) and a scan of the lengths into start bits
+        // the run values (into LDS) and a scan of the lengths into start bits.
+        // The next batch's words are loaded while a batch is worked on.
+        auto fetch = [&](uint64_t i0, uint32_t (&wv8)[K]) {
+            if (i0 + K <= avail) {
+#pragma unroll
+                for (int q = 0; q < K / 4; q++) {
+                    const Words4 v = *reinterpret_cast<const Words4 *>(wd + i0 + 4 * q);
+#pragma unroll
+                    for (int j = 0; j < 4; j++) wv8[4 * q + j] = v.w[j];
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < K; j++) wv8[j] = (i0 + j < avail) ? wd[i0 + j] : 1u;
+            }
+        };
         uint64_t pos = 0;
+        uint32_t cur[K], par = 0;
+        if (nz) fetch((uint64_t)threadIdx.x * K, cur);
         for (uint64_t b0 = 0; b0 < nz; b0 += (uint64_t)BS * K) {
             const uint64_t i0 = b0 + (uint64_t)threadIdx.x * K;
-            uint32_t wv[K];
+            uint32_t nxt[K] = {};
+            if (b0 + (uint64_t)BS * K < nz) fetch(i0 + (uint64_t)BS * K, nxt);
+            uint32_t len[K];
+            uint64_t st = 0;
+            uint32_t tot = 0;
+            for (;;) {
+                uint32_t lsum = 0;
+                bool bad = false;
 #pragma unroll
-            for (int j = 0; j < K; j++) wv[j] = (i0 + j < avail) ? wd[i0 + j] : 1u;
+                for (int j = 0; j < K; j++) {
+                    const uint64_t i = i0 + j;
+                    uint32_t l = (i < nz) ? (cur[j] & 0xFFFFFFu) : 0u;
+                    // a 0 word before the known end is the end
+                    if (cur[j] == 0u && i >= 1 && i < nz && i <= 0xFFFFFFFFull)
+                        atomicMin(&s_nz, (uint32_t)i);
+                    bad |= (i < nz) && (l == 0u || l > LMAX);   // zero-length or oversized runs
+                    l = l < LMAX ? l : LMAX;
+                    len[j] = l;
+                    lsum += l;
+                }
+                uint32_t wt;
+                const uint32_t ex = wave_excl_scan(lsum, wt);
+                if (ln == 0) wtot[par * NW + wv] = wt;
+                __syncthreads();
+                // a wave ahead of this one may have met an end in the next batch
+                const uint64_t end = s_nz, stop = min(nz, b0 + (uint64_t)BS * K);
+                uint32_t before = 0;
+                tot = 0;
 #pragma unroll
-            for (int j = 0; j < K; j++)
-                if (i0 + j >= 1 && i0 + j < avail && i0 + j <= 0xFFFFFFFFull && wv[j] == 0u)
-                    atomicMin(&s_nz, (uint32_t)(i0 + j));
-            __syncthreads();
-            nz = s_nz;
-            uint32_t len[K], lsum = 0;
-            bool bad = false;
+                for (int q = 0; q < NW; q++) {
+                    const uint32_t t = wtot[par * NW + q];
+                    before += q < wv ? t : 0u;
+                    tot += t;
+                }
+                par ^= 1u;
+                st = pos + before + ex;
+                if (end < stop && end < 0xFFFFFFFFull) {   // uniform: an early end
+                    nz = end;
+                    continue;
+                }
+                if (bad) s_bad = 1u;
+                break;
+            }
 #pragma unroll
             for (int j = 0; j < K; j++) {
                 const uint64_t i = i0 + j;
-                uint32_t l = (i < nz) ? (wv[j] & 0xFFFFFFu) : 0u;
-                bad |= (i < nz) && (l == 0u || l > LMAX);   // zero-length or oversized runs
-                l = l < LMAX ? l : LMAX;
-                len[j] = l;
-                lsum += l;
-                if (i < nz && i < (uint64_t)VCAP) val8[i] = (uint8_t)(wv[j] >> 24);
+                if (i < nz && i < (uint64_t)VCAP) val8[i + 1] = (uint8_t)(cur[j] >> 24);
             }
-            if (bad) s_bad = 1u;
-            uint32_t tot = 0;
-            uint64_t st = pos + r_scan_excl<BS>(lsum, wsum, tot);
+            // the starts of a 32-bit word of the map go there together
+            uint32_t at = 0, bits = 0;
 #pragma unroll
             for (int j = 0; j < K; j++) {
-                if (len[j] && st < (uint64_t)VOX)
-                    atomicOr(reinterpret_cast<unsigned long long *>(&bm[st >> 6]), 1ull << (st & 63u));
+                if (len[j] && st < (uint64_t)VOX) {
+                    const uint32_t w = (uint32_t)st >> 5;
+                    if (w != at) {
+                        if (bits) atomicOr(&bm32[at], bits);
+                        at = w;
+                        bits = 0;
+                    }
+                    bits |= 1u << ((uint32_t)st & 31u);
+                }
                 st += len[j];
             }
+            if (bits) atomicOr(&bm32[at], bits);
             pos += tot;
+#pragma unroll
+            for (int j = 0; j < K; j++) cur[j] = nxt[j];
         }
         if (threadIdx.x == 0 && pos != (uint64_t)VOX) s_bad = 1u;
         __syncthreads();
         const uint64_t nw = nz;
-        // rank of each bitmap word = starts before it
-        uint32_t mine = 0;
-        const int w0 = (int)threadIdx.x * WPT;
-        for (int j = 0; j < WPT; j++)
-            if (w0 + j < WORDS) mine += (uint32_t)__popcll(bm[w0 + j]);
-        uint32_t tot = 0;
-        uint32_t run = r_scan_excl<BS>(mine, wsum, tot);
-        for (int j = 0; j < WPT; j++)
-            if (w0 + j < WORDS) {
-                rank[w0 + j] = run;
-                run += (uint32_t)__popcll(bm[w0 + j]);
+        // rank of each bitmap word = starts before it: words strided over the
+        // threads, a scan per wave and row of words, then one of the totals
+        uint32_t rk[WPT];
+#pragma unroll
+        for (int j = 0; j < WPT; j++) {
+            const int w = j * BS + (int)threadIdx.x;
+            const uint32_t c = w < WORDS ? (uint32_t)__popcll(bm[w]) : 0u;
+            uint32_t wt;
+            rk[j] = wave_excl_scan(c, wt);
+            if (ln == 0) wtot[j * NW + wv] = wt;
+        }
+        __syncthreads();
+        {
+            uint32_t all;
+            const uint32_t t = wave_excl_scan((int)ln < WPT * NW ? wtot[ln] : 0u, all);
+#pragma unroll
+            for (int j = 0; j < WPT; j++) {
+                const int w = j * BS + (int)threadIdx.x;
+                const uint32_t base = (uint32_t)__builtin_amdgcn_readlane((int)t, j * NW + wv);
+                if (w < WORDS) rank[w] = base + rk[j];
             }
+        }
         __syncthreads();
         // bytes: run index of byte p = starts at or before p, minus one; each
-        // start belongs to a run index below nw
+        // start belongs to a run index below nw.  A piece of 16 bytes with up
+        // to 7 starts takes its values from 8 consecutive bytes, picked by the
+        // running count of its starts: four counts at a time from a multiply
+        // and two adds, one byte permute per four bytes.
         const bool in_lds = nw <= (uint64_t)VCAP;
-        for (int s = threadIdx.x; s < VOX / 16; s += BS) {
+        for (int s = p_lo + (int)threadIdx.x; s < p_hi; s += BS) {
             const int w = s >> 2;
             const uint64_t b = bm[w];
+            if ((s & 3) == 3) bm[w] = 0ull;     // cleared for the next chunk: its four readers are this wave's
             const int sh = (s & 3) * 16;
-            const uint64_t below = sh ? (b & ((1ull << sh) - 1ull)) : 0ull;
-            const int r0 = (int)(rank[w] + (uint32_t)__popcll(below)) - 1;
+            const uint64_t below = b & ((1ull << sh) - 1ull);
+            const uint32_t idx = rank[w] + (uint32_t)__popcll(below);   // run index + 1 of byte -1
             const uint32_t bits16 = (uint32_t)(b >> sh) & 0xFFFFu;
             uint32_t out[4] = {0, 0, 0, 0};
             const uint64_t p0 = (uint64_t)s * 16;
+            if (in_lds && p0 + 16 <= pos && __popc(bits16) <= 7) {
+                const uint32_t *v = val32 + (idx >> 2);
+                const uint32_t v0 = v[0], v1 = v[1], v2 = v[2];
+                const uint32_t lo = __builtin_amdgcn_alignbyte(v1, v0, idx & 3u);
+                const uint32_t hi = __builtin_amdgcn_alignbyte(v2, v1, idx & 3u);
+                uint32_t base = 0;              // starts so far, in each byte
 #pragma unroll
-            for (int j = 0; j < 16; j++) {
-                const int ri = r0 + __popc(bits16 & ((2u << j) - 1u));
-                uint32_t v = 0;
-                if (ri >= 0 && p0 + j < pos) v = in_lds ? (uint32_t)val8[ri] : (wd[ri] >> 24);
-                out[j >> 2] |= v << ((j & 3) * 8);
+                for (int d = 0; d < 4; d++) {
+                    uint32_t t = __umul24((bits16 >> (4 * d)) & 15u, 0x204081u) & 0x01010101u;
+                    t += t << 8;
+                    t += t << 16;               // byte j: starts in bytes 0..j
+                    t += base;
+                    out[d] = __builtin_amdgcn_perm(hi, lo, t);
+                    base = __builtin_amdgcn_perm(t, t, 0x03030303u);
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 16; j++) {
+                    const int ri = (int)idx - 1 + __popc(bits16 & ((2u << j) - 1u));
+                    uint32_t v = 0;
+                    if (ri >= 0 && p0 + j < pos)
+                        v = in_lds ? (uint32_t)val8[ri + 1] : (wd[ri] >> 24);
+                    out[j >> 2] |= v << ((j & 3) * 8);
+                }
             }
             nt_store16(dst + p0, make_uint4(out[0], out[1], out[2], out[3]));
         }
@@ -538,6 +653,7 @@ extern "C" int vp_gpu_rle(vp_ctx *ctx, int dir, const vp_world_desc *world,
     a.uniform_out = d_uniform_out;
     a.status = ctx->d_status;
     a.single = (n == 1) ? 1 : 0;
+    a.parts = 1u;
     a.nchunks = (uint32_t)(1ull << (world->max_bitw[0] + world->max_bitw[1] + world->max_bitw[2]));
     int grid = 1;
     if (dir == VP_RLE_ENCODE) {
@@ -555,8 +671,13 @@ extern "C" int vp_gpu_rle(vp_ctx *ctx, int dir, const vp_world_desc *world,
             VP_HIP_TRY(hipGetLastError());
         }
     } else {
-        const int resident = ctx->num_cus * 2;
-        grid = (int)(n < (uint32_t)resident ? n : (uint32_t)resident);
+        const uint32_t resident = (uint32_t)ctx->num_cus * 2u;
+        // Few 64^3 chunks: up to eight workgroups repeat a chunk's scan and
+        // share out its bytes, as many as fit at once (two chunks: 50 -> 26 us
+        // by one workgroup each, 18 us by eight; smaller edges are done
+        // within a launch's latency).
+        while (root_bitw == 6 && a.parts < 8u && (uint64_t)n * a.parts * 2u <= resident) a.parts *= 2u;
+        grid = (int)(n < resident ? n * a.parts : resident);
     }
     return rle_dispatch(root_bitw, dir, a, grid, st) == hipSuccess ? VP_OK : VP_ERR_HIP;
 }

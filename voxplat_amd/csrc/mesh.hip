@@ -30,6 +30,7 @@
 #include "vp_internal.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace vp {
 
@@ -72,22 +73,59 @@ __device__ __forceinline__ uint32_t m_corner(uint32_t axis, uint32_t v)
     return (w >> (3 * v)) & 7u;
 }
 
-// triangle index rows by [normal][rotated] (mesher.c:54-66), 2 bits each
-__device__ __forceinline__ uint32_t m_tri(uint32_t normal, uint32_t rot, uint32_t k)
+// triangle index rows by normal | rotated << 1 (mesher.c:54-66), 2 bits each
+__device__ __forceinline__ uint32_t m_tri_row(uint32_t normal, uint32_t rot)
 {
     constexpr uint32_t r00 = 0u | 3u << 2 | 1u << 4 | 2u << 6 | 1u << 8 | 3u << 10;
     constexpr uint32_t r01 = 3u | 2u << 2 | 0u << 4 | 1u << 6 | 0u << 8 | 2u << 10;
     constexpr uint32_t r10 = 1u | 3u << 2 | 0u << 4 | 3u << 6 | 1u << 8 | 2u << 10;
     constexpr uint32_t r11 = 0u | 2u << 2 | 3u << 4 | 2u << 6 | 0u << 8 | 1u << 10;
-    const uint32_t row = normal ? (rot ? r11 : r10) : (rot ? r01 : r00);
-    return (row >> (2 * k)) & 3u;
+    return normal ? (rot ? r11 : r10) : (rot ? r01 : r00);
 }
+
+// Vertex ambient terms, 2 bits each in vertex order, and the rotated flag at
+// bit 8, of a face whose air cell has the in-plane neighbours nb: bit
+// 3 (1 + d1) + 1 + d0 for the step d0 along the lower and d1 along the higher
+// of the face's two axes (sample_ao, mesher.c:72-171, vertex order of
+// mesher.c:254-272).
+constexpr uint32_t m_ambient(uint32_t axis, uint32_t nb)
+{
+    auto at = [&](int d0, int d1) -> uint32_t { return (nb >> (3 * (1 + d1) + 1 + d0)) & 1u; };
+    const uint32_t n0 = at(-1, 0), n1 = at(0, -1), n2 = at(1, 0), n3 = at(0, 1);
+    const uint32_t c0 = (n0 + n1) | at(-1, -1), c1 = (n1 + n2) | at(1, -1);
+    const uint32_t c2 = (n2 + n3) | at(1, 1), c3 = (n3 + n0) | at(-1, 1);
+    const uint32_t v0 = axis == 2 ? c1 : c0, v2 = axis == 2 ? c3 : c2;
+    const uint32_t v1 = axis == 0 ? c3 : (axis == 1 ? c1 : c0);
+    const uint32_t v3 = axis == 0 ? c1 : (axis == 1 ? c3 : c2);
+    return v0 | v1 << 2 | v2 << 4 | v3 << 6 | (v0 + v2 < v1 + v3 ? 1u : 0u) << 8;
+}
+
+// m_ambient of all axes and neighbours, two 16-bit entries to a word
+struct AmbientTable {
+    uint32_t w[3 * 256];
+};
+constexpr AmbientTable ambient_table()
+{
+    AmbientTable t = {};
+    for (uint32_t i = 0; i < 3 * 256; i++)
+        t.w[i] = m_ambient(i >> 8, 2 * i & 511u) | m_ambient(i >> 8, (2 * i + 1) & 511u) << 16;
+    return t;
+}
+__constant__ const AmbientTable kAmbient = ambient_table();
 
 // 16 bytes -> 16 occupancy bits
 __device__ __forceinline__ uint32_t nz4(uint32_t w)
 {
     const uint32_t m = (((w & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | w) & 0x80808080u;
     return (((m >> 7) * 0x00204081u) >> 21) & 0xFu;
+}
+
+// sums of the two 16-bit halves
+__device__ __forceinline__ uint32_t add_u16x2(uint32_t a, uint32_t b)
+{
+    typedef unsigned short v2 __attribute__((ext_vector_type(2)));
+    const v2 s = __builtin_bit_cast(v2, a) + __builtin_bit_cast(v2, b);
+    return __builtin_bit_cast(uint32_t, s);
 }
 
 template <int B>
@@ -97,8 +135,8 @@ struct MeshShape {
     static constexpr int ROWS = R * R;                     // (z, y) rows of the chunk
     static constexpr int GR = ROWS >= kMeshBS ? ROWS / kMeshBS : 1;   // rows per group
     static constexpr int NG = ROWS / GR;                   // groups (one per thread)
-    static constexpr int LIST = 3 * R * R * R < 4096 ? 3 * R * R * R : 4096;   // faces per pass
-    static constexpr int KF = (LIST + kMeshBS - 1) / kMeshBS;   // faces per thread per pass
+    static constexpr int LIST = 3 * R * R * R < 2048 ? 3 * R * R * R : 2048;   // faces per pass
+    static constexpr int W = (R + 2 + 31) / 32;            // words of a row with its shell
     static constexpr int QW = R >= 16 ? 16 : R;            // bytes per row load
     static constexpr int Q = R / QW;                       // loads per row
     static constexpr uint64_t FULL = R == 64 ? ~0ull : ((1ull << R) - 1ull);
@@ -126,142 +164,103 @@ template <int BS>
 __device__ __forceinline__ uint32_t m_scan_excl(uint32_t v, uint32_t *wsum, uint32_t &total)
 {
     constexpr int NW = BS / 64;
-    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
-    uint32_t x = v;
+    const uint32_t w = threadIdx.x >> 6;
+    uint32_t wt, before = 0;
+    const uint32_t ex = wave_excl_scan(v, wt);
+    if ((threadIdx.x & 63u) == 0) wsum[w] = wt;
+    __syncthreads();
+    total = 0;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t y = __shfl_up(x, d, 64);
-        if (lane >= (uint32_t)d) x += y;
+    for (uint32_t i = 0; i < NW; i++) {
+        before += i < w ? wsum[i] : 0u;
+        total += wsum[i];
     }
-    if (lane == 63) wsum[w] = x;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t run = 0;
-        for (int i = 0; i < NW; i++) {
-            const uint32_t t = wsum[i];
-            wsum[i] = run;
-            run += t;
-        }
-        wsum[NW] = run;
-    }
-    __syncthreads();
-    total = wsum[NW];
-    const uint32_t r = wsum[w] + x - v;
-    __syncthreads();
-    return r;
+    return before + ex;
 }
 
-// per-face state between the LDS work and the global loads: the colour
-// byte's address (null: the colour is in meta), the shadow-map entry i the
-// face's samples are centred on, the voxel's y, and
-// meta = colour | axis << 8 | vao << 10 | rot << 18 | valid << 19 |
-//        (reads i - 1) << 20 | (reads i + 1) << 21 | (reads i) << 22
-struct FaceWork {
-    const uint8_t *cptr;
-    uint32_t mi;
-    uint32_t wy;
-    uint32_t meta;
-};
-
-// LDS half of one face of the list: the air cell's in-plane neighbours give
-// the vertex ambient terms (sample_ao, mesher.c:72-171, and the vertex order
-// of mesher.c:254-272), and the addresses of the colour byte and the shadow
-// map entries the face needs (mesher.c:282-320, shadow.h:52-75)
+// An occupancy row: bit x + 1 is voxel x, bits 0 and R + 1 the shell.
 template <int B>
-__device__ __forceinline__ void prep_face(FaceWork &w, uint32_t j, uint32_t pf, const uint32_t *list,
-                                          const uint64_t *occ, const uint8_t *edge, const int16_t *s_uni,
-                                          const uint32_t *s_nid, const uint8_t *voxels, uint32_t map_sx,
-                                          uint32_t ox, uint32_t oy, uint32_t oz)
+__device__ __forceinline__ uint64_t row_from(const uint32_t *w, int sh)
 {
-    constexpr int R = 1 << B, P = R + 2;
-    const uint32_t e = list[j < pf ? j : 0u];
-    const uint32_t axis = e & 3u, x = (e >> 2) & 63u, r = e >> 8;
-    const int z = (int)(r >> B), yl = (int)(r & (R - 1));
-    const int r0 = (z + 1) * P + (yl + 1);
-    const uint32_t solid_a = (uint32_t)(occ[r0] >> x) & 1u;
-    // the air cell of the pair (A itself, or B when A is solid)
-    const int px = (int)x + (axis == 0 ? (int)solid_a : 0);
-    const int py = yl + (axis == 1 ? (int)solid_a : 0);
-    const int pz = z + (axis == 2 ? (int)solid_a : 0);
-    // occupancy at shell coordinates in [-1, R]; both words are read and the
-    // bit selected without a branch, so the eight samples' reads issue together
-    auto sol = [&](int qx, int qy, int qz) -> uint32_t {
-        const int rr = (qz + 1) * P + (qy + 1);
-        const uint64_t rw = occ[rr];
-        const uint32_t eg = edge[rr];
-        const uint32_t in = (uint32_t)(rw >> (qx & 63)) & 1u;
-        const uint32_t m_lo = 0u - (uint32_t)(qx < 0), m_hi = 0u - (uint32_t)(qx >= R);
-        return (in & ~(m_lo | m_hi)) | (eg & m_lo & 1u) | ((eg >> 1) & m_hi);
-    };
-    // steps d0 along u0 and d1 along u1, the two axes other than the
-    // face's, in ascending order
-    auto at = [&](int d0, int d1) -> uint32_t {
-        return sol(px + (axis != 0 ? d0 : 0), py + (axis == 0 ? d0 : (axis == 2 ? d1 : 0)),
-                   pz + (axis != 2 ? d1 : 0));
-    };
-    const uint32_t n0 = at(-1, 0), n1 = at(0, -1), n2 = at(1, 0), n3 = at(0, 1);
-    const uint32_t c0 = (n0 + n1) | at(-1, -1);
-    const uint32_t c1 = (n1 + n2) | at(1, -1);
-    const uint32_t c2 = (n2 + n3) | at(1, 1);
-    const uint32_t c3 = (n3 + n0) | at(-1, 1);
-    uint32_t v0, v1, v2, v3;
+    using S = MeshShape<B>;
+    if constexpr (S::W == 3)
+        return (uint64_t)__builtin_amdgcn_alignbit(w[2], w[1], sh) << 32 |
+               __builtin_amdgcn_alignbit(w[1], w[0], sh);
+    else if constexpr (S::W == 2)
+        return __builtin_amdgcn_alignbit(w[1], w[0], sh);
+    else
+        return (w[0] >> sh) & (uint32_t)S::FULL;
+}
+// voxels x = 0..R-1 as bits, and the same of their +x neighbours
+template <int B>
+__device__ __forceinline__ uint64_t row_own(const uint32_t *w) { return row_from<B>(w, 1); }
+template <int B>
+__device__ __forceinline__ uint64_t row_next(const uint32_t *w) { return row_from<B>(w, 2); }
+
+// The nine occupancy bits around the air cell (px, py, pz) in the face's plane,
+// as m_ambient takes them: three bits of three rows for y and z faces, one bit
+// of nine rows for x faces.
+template <int B>
+__device__ __forceinline__ uint32_t plane_bits(const uint32_t *occ, uint32_t axis, int px, int py, int pz)
+{
+    constexpr int P = MeshShape<B>::P, W = MeshShape<B>::W;
+    const int row = (pz + 1) * P + (py + 1);
+    uint32_t nb = 0;
     if (axis == 0) {
-        v0 = c0; v3 = c1; v2 = c2; v1 = c3;
-    } else if (axis == 1) {
-        v0 = c0; v1 = c1; v2 = c2; v3 = c3;
+        const uint32_t ix = (uint32_t)px + 1u;
+        const uint32_t *w = occ + (row - P - 1) * W + (ix >> 5);
+#pragma unroll
+        for (int d1 = 0; d1 < 3; d1++)
+#pragma unroll
+            for (int d0 = 0; d0 < 3; d0++)
+                nb |= ((w[(d1 * P + d0) * W] >> (ix & 31u)) & 1u) << (3 * d1 + d0);
     } else {
-        v1 = c0; v0 = c1; v3 = c2; v2 = c3;
+        const uint32_t ix = (uint32_t)px;              // bits px - 1 .. px + 1
+        const int step = (axis == 1 ? P : 1) * W;
+        const uint32_t *w = occ + row * W - step + (ix >> 5);
+#pragma unroll
+        for (int d1 = 0; d1 < 3; d1++)
+            nb |= (__builtin_amdgcn_alignbit(w[d1 * step + 1], w[d1 * step], ix & 31u) & 7u) << (3 * d1);
     }
-    const uint32_t rot = (v0 + v2 < v1 + v3) ? 1u : 0u;
-    const uint32_t vao = v0 | v1 << 2 | v2 << 4 | v3 << 6;
-    const uint32_t valid = j < pf ? 1u : 0u;
-    const uint32_t wx = ox + x, wy = oy + (uint32_t)yl, wz = oz + (uint32_t)z;
-    // the solid voxel of the pair: A, or B at +axis (maybe in the next chunk)
-    const uint32_t bx = x + (axis == 0), by = (uint32_t)yl + (axis == 1), bz = (uint32_t)z + (axis == 2);
-    const uint32_t sx = solid_a ? x : bx, sy = solid_a ? (uint32_t)yl : by, sz = solid_a ? (uint32_t)z : bz;
-    const int nb = 13 + (sx >= (uint32_t)R) + 3 * (sy >= (uint32_t)R) + 9 * (sz >= (uint32_t)R);
-    const int16_t un = s_uni[nb];
-    const uint32_t cval = un >= 0 ? (uint32_t)un : 0u;
-    w.cptr = un >= 0 ? nullptr
-                     : voxels + ((uint64_t)s_nid[nb] << (3 * B)) +
-                           ((((sz & (R - 1)) << B | (sy & (R - 1))) << B) | (sx & (R - 1)));
-    // shadow samples: entries (i, i - 1) of the solid +x cell for x faces of
-    // air; (i, i + 1) of the voxel for y faces of solid voxels; for z faces
-    // (i, i + 1) of the cell in front and (i - 1, i) one below it
-    uint32_t need = 0;
-    w.mi = 0;
-    if (axis == 0 && !solid_a) {
-        w.mi = (wx + 1u + wy) + map_sx * wz;
-        need = 1u << 20 | 1u << 22;
-    } else if (axis == 1 && solid_a) {
-        w.mi = (wx + wy) + map_sx * wz;
-        need = 1u << 21 | 1u << 22;
-    } else if (axis == 2) {
-        w.mi = (wx + wy) + map_sx * (wz + solid_a);
-        need = (wy != 0u ? 1u << 20 : 0u) | 1u << 21 | 1u << 22;
-    }
-    w.wy = wy;
-    w.meta = cval | axis << 8 | vao << 10 | rot << 18 | valid << 19 | (valid ? need : 0u);
+    return nb;
 }
 
 template <int B>
 __global__ void __launch_bounds__(kMeshBS, 4) k_mesh(MeshArgs a)
 {
     using S = MeshShape<B>;
-    constexpr int R = S::R, P = S::P, BS = kMeshBS, KF = S::KF;
+    constexpr int R = S::R, P = S::P, W = S::W, BS = kMeshBS;
     using RL = RowLoad<S::QW>;
-    __shared__ uint64_t occ[P * P];          // bits x = 0..R-1 of row (z, y), shell coordinates + 1
-    __shared__ uint8_t  edge[P * P];         // bit 0: x = -1, bit 1: x = R
+    __shared__ uint32_t occ[P * P * W + 2];  // row (z, y) in shell coordinates + 1, bits as row_own
     __shared__ uint8_t  rowcnt[S::ROWS];     // faces of each chunk row
     __shared__ uint32_t goff[S::NG + 1];     // face offset of each row group
-    __shared__ uint32_t list[S::LIST];       // (row << 8 | x << 2 | axis) of a pass's faces
-    __shared__ uint32_t wsum[BS / 64 + 1];
+    __shared__ uint32_t list[S::LIST];       // solid << 20 | row << 8 | x << 2 | axis of a pass's faces
+    __shared__ uint32_t packed[S::LIST];     // and all else their vertices and indices take
+    __shared__ uint32_t wsum[BS / 64];
+    __shared__ AmbientTable s_amb;           // u16 by axis << 9 | plane bits
+    __shared__ uint4    s_corner[6];         // per axis and half: two vertices' (xy, z | number << 27)
     __shared__ int16_t  s_uni[27];           // 3x3x3 neighbourhood: value if uniform (0 = air/outside), -1 mixed
     __shared__ uint32_t s_nid[27];
     __shared__ uint32_t s_ticket;
     __shared__ uint64_t s_base;
 
     const uint32_t mx = 1u << a.mb0, my = 1u << a.mb1, mz = 1u << a.mb2;
+    // the ambient table on its way to LDS, stored there by the first visit
+    constexpr int TW = (3 * 256 + BS - 1) / BS;
+    uint32_t tab[TW] = {};
+    if (a.geom) {
+        for (int i = 0; i < TW; i++)
+            if (i * BS + threadIdx.x < 3u * 256u) tab[i] = kAmbient.w[i * BS + threadIdx.x];
+        if (threadIdx.x < 6) {
+            uint32_t w[4];
+            for (uint32_t h = 0; h < 2; h++) {
+                const uint32_t v = 2u * (threadIdx.x & 1u) + h, c = m_corner(threadIdx.x >> 1, v);
+                w[2 * h] = (c & 1u) | ((c >> 1) & 1u) << 16;
+                w[2 * h + 1] = (c >> 2) | v << 27;
+            }
+            s_corner[threadIdx.x] = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+    }
     for (uint32_t visit = 0;; visit++) {
         // a single chunk takes no ticket: workgroup p does part p of list entry 0
         if (threadIdx.x == 0)
@@ -326,9 +325,16 @@ __global__ void __launch_bounds__(kMeshBS, 4) k_mesh(MeshArgs a)
 #pragma unroll
                         for (int d = 1; d < S::Q; d <<= 1) r |= __shfl_xor(r, d, 64);
                     }
-                    if (t < NI && t % S::Q == 0) occ[t / S::Q] = r;
+                    if (t < NI && t % S::Q == 0) {
+                        uint32_t *w = occ + t / S::Q * W;
+                        w[0] = (uint32_t)r << 1;
+                        if constexpr (W > 1) w[1] = (uint32_t)(r >> 31);
+                        if constexpr (W > 2) w[2] = (uint32_t)(r >> 63);
+                    }
                 }
             }
+            __syncthreads();
+            // the shell's x = -1 and x = R
             constexpr int NE = P * P, UE = 3;
             for (int t0 = threadIdx.x; t0 < NE; t0 += UE * BS) {
                 uint8_t lo[UE], hi[UE];
@@ -343,16 +349,19 @@ __global__ void __launch_bounds__(kMeshBS, 4) k_mesh(MeshArgs a)
                         const uint64_t ro = ((((uint64_t)((uint32_t)(zz - 1) & (R - 1))) << B) |
                                              ((uint32_t)(yy - 1) & (R - 1))) << B;
                         const int16_t ul = s_uni[nb - 1], uh = s_uni[nb + 1];
-                        lo[u] = ul >= 0 ? (ul != 0)
-                                        : (a.voxels[((uint64_t)s_nid[nb - 1] << (3 * B)) + ro + (R - 1)] != 0);
-                        hi[u] = uh >= 0 ? (uh != 0)
-                                        : (a.voxels[((uint64_t)s_nid[nb + 1] << (3 * B)) + ro] != 0);
+                        lo[u] = ul >= 0 ? (uint8_t)(ul != 0)
+                                        : a.voxels[((uint64_t)s_nid[nb - 1] << (3 * B)) + ro + (R - 1)];
+                        hi[u] = uh >= 0 ? (uint8_t)(uh != 0)
+                                        : a.voxels[((uint64_t)s_nid[nb + 1] << (3 * B)) + ro];
                     }
                 }
 #pragma unroll
                 for (int u = 0; u < UE; u++) {
                     const int row = t0 + u * BS;
-                    if (row < NE) edge[row] = (uint8_t)(lo[u] | hi[u] << 1);
+                    if (row < NE) {
+                        if (lo[u]) occ[row * W] |= 1u;
+                        if (hi[u]) occ[row * W + (R + 1) / 32] |= 1u << ((R + 1) % 32);
+                    }
                 }
             }
         }
@@ -365,17 +374,19 @@ __global__ void __launch_bounds__(kMeshBS, 4) k_mesh(MeshArgs a)
             for (int i = 0; i < S::GR; i++) {
                 const int r = threadIdx.x * S::GR + i;
                 const int z = r / R, y = r % R;
-                const int r0 = (z + 1) * P + (y + 1);
-                const uint64_t o = occ[r0];
-                const uint64_t bx = (o >> 1) | ((uint64_t)(edge[r0] >> 1) << (R - 1));
-                const uint32_t c = __popcll((o ^ bx) & S::FULL) + __popcll((o ^ occ[r0 + 1]) & S::FULL) +
-                                   __popcll((o ^ occ[r0 + P]) & S::FULL);
+                const uint32_t *w = occ + ((z + 1) * P + (y + 1)) * W;
+                const uint64_t o = row_own<B>(w);
+                const uint32_t c = __popcll(o ^ row_next<B>(w)) + __popcll(o ^ row_own<B>(w + W)) +
+                                   __popcll(o ^ row_own<B>(w + P * W));
                 rowcnt[r] = (uint8_t)c;
                 gcnt += c;
             }
         }
         uint32_t faces;
         const uint32_t gex = m_scan_excl<BS>(gcnt, wsum, faces);
+        if (a.geom && visit == 0)
+            for (int i = 0; i < TW; i++)
+                if (i * BS + threadIdx.x < 3u * 256u) s_amb.w[i * BS + threadIdx.x] = tab[i];
         if (threadIdx.x < S::NG) goff[threadIdx.x] = gex;
         if (threadIdx.x == 0) goff[S::NG] = faces;
         if (threadIdx.x < 64) {
@@ -423,6 +434,8 @@ __global__ void __launch_bounds__(kMeshBS, 4) k_mesh(MeshArgs a)
 
         // ---- 3./4. faces, in passes of whole row groups that fit the list ----
         const uint32_t ox = cx << B, oy = cy << B, oz = cz << B;
+        const int16_t own_u = s_uni[13];
+        const uint8_t *own = a.voxels + ((uint64_t)id << (3 * B));
         // this part's row groups: those whose first face lies in its share
         uint32_t g0 = 0, gend = (uint32_t)S::NG;
         if (a.parts > 1u) {
@@ -452,22 +465,21 @@ __global__ void __launch_bounds__(kMeshBS, 4) k_mesh(MeshArgs a)
                     uint32_t pos = goff[g] - lo;
                     for (uint32_t q = g * S::GR; q < r; q++) pos += rowcnt[q];
                     const int z = (int)(r / R), y = (int)(r % R);
-                    const int r0 = (z + 1) * P + (y + 1);
-                    const uint64_t o = occ[r0];
-                    const uint64_t bx = (o >> 1) | ((uint64_t)(edge[r0] >> 1) << (R - 1));
-                    const uint64_t fx = (o ^ bx) & S::FULL, fy = (o ^ occ[r0 + 1]) & S::FULL,
-                                   fz = (o ^ occ[r0 + P]) & S::FULL;
+                    const uint32_t *w = occ + ((z + 1) * P + (y + 1)) * W;
+                    const uint64_t o = row_own<B>(w);
+                    const uint64_t fx = o ^ row_next<B>(w), fy = o ^ row_own<B>(w + W),
+                                   fz = o ^ row_own<B>(w + P * W);
                     const uint32_t sh = sg * SW;
                     const uint64_t below = (1ull << sh) - 1ull;
                     pos += __popcll(fx & below) + __popcll(fy & below) + __popcll(fz & below);
                     constexpr uint32_t SM = (1u << SW) - 1u;
                     const uint32_t mxb = (uint32_t)(fx >> sh) & SM, myb = (uint32_t)(fy >> sh) & SM,
-                                   mzb = (uint32_t)(fz >> sh) & SM;
+                                   mzb = (uint32_t)(fz >> sh) & SM, ob = (uint32_t)(o >> sh) & SM;
                     uint32_t any = mxb | myb | mzb;
                     while (any) {
                         const uint32_t j = (uint32_t)__builtin_ctz(any);
                         any &= any - 1u;
-                        const uint32_t e = r << 8 | (sh + j) << 2;
+                        const uint32_t e = ((ob >> j) & 1u) << 20 | r << 8 | (sh + j) << 2;
                         if ((mxb >> j) & 1u) list[pos++] = e | 0u;
                         if ((myb >> j) & 1u) list[pos++] = e | 1u;
                         if ((mzb >> j) & 1u) list[pos++] = e | 2u;
@@ -477,86 +489,101 @@ __global__ void __launch_bounds__(kMeshBS, 4) k_mesh(MeshArgs a)
             __syncthreads();
             // E1: everything but the stores -- ambient terms from LDS, the
             // colour byte and the shadow samples from memory -- packed into
-            // one word per face; E2: the stores only, so no load waits behind
-            // them (vector memory counters retire loads and stores in order)
-            uint32_t packed[KF];
+            // one word per face: the vertices' common attribute bits below,
+            // then the ambient terms and the rotated flag
+            auto prepare = [&](auto uc, uint32_t j0) {
+                constexpr int U = decltype(uc)::value;      // faces of a thread in flight
+                uint32_t amb[U], col[U], cval[U], pair[U], pair2[U], e[U], wy[U];
 #pragma unroll
-            for (int k0 = 0; k0 < KF; k0 += 2) {
-                if (threadIdx.x + (uint32_t)k0 * BS >= pf) break;
-                FaceWork fw[2];
-#pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    if (k0 + u < KF)
-                        prep_face<B>(fw[u], threadIdx.x + (uint32_t)(k0 + u) * BS, pf, list, occ, edge,
-                                     s_uni, s_nid, a.voxels, a.map_sx, ox, oy, oz);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                uint32_t col[2], elo[2], emid[2], ehi[2];
-#pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    if (k0 + u >= KF) break;
-                    const FaceWork &w = fw[u];
-                    col[u] = ((w.meta >> 19) & 1u) && w.cptr ? (uint32_t)*w.cptr : (w.meta & 0xFFu);
-                    elo[u] = ((w.meta >> 20) & 1u) ? a.map[w.mi - 1u] : 0u;
-                    emid[u] = ((w.meta >> 22) & 1u) ? a.map[w.mi] : 0u;
-                    ehi[u] = ((w.meta >> 21) & 1u) ? a.map[w.mi + 1u] : 0u;
-                }
-#pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    if (k0 + u >= KF) break;
-                    const FaceWork &w = fw[u];
-                    const uint32_t axis = (w.meta >> 8) & 3u, top = w.wy + 1u;
-                    uint32_t shadow = 0, diamond = 3;
-                    if ((w.meta >> 22) & 1u) {
-                        if (axis == 0) {
-                            shadow = (emid[u] < top && elo[u] < top) ? 0u : 1u;
-                        } else if (axis == 1) {
-                            shadow = (emid[u] < top && ehi[u] < top) ? 0u : 1u;
-                        } else {
-                            const uint32_t lit0 = (emid[u] < top && ehi[u] < top) ? 1u : 0u;
-                            const uint32_t lit1 = (w.wy != 0u && elo[u] < w.wy && emid[u] < w.wy) ? 1u : 0u;
-                            diamond = lit0 << 1 | lit1;
-                        }
+                for (int u = 0; u < U; u++) {
+                    e[u] = list[min(j0 + (uint32_t)u * BS, pf - 1u)];
+                    const uint32_t axis = e[u] & 3u, x = (e[u] >> 2) & 63u, r = (e[u] >> 8) & 4095u;
+                    const uint32_t solid = e[u] >> 20, air = solid ^ 1u;
+                    const uint32_t z = r >> B, yl = r & (R - 1);
+                    const uint32_t ax = axis == 0, ay = axis == 1, az = axis == 2;
+                    // the air cell of the pair is A, or B when A is solid
+                    const uint32_t nb = plane_bits<B>(occ, axis, (int)(x + (ax & solid)),
+                                                      (int)(yl + (ay & solid)), (int)(z + (az & solid)));
+                    amb[u] = reinterpret_cast<const uint16_t *>(s_amb.w)[axis << 9 | nb];
+                    // the solid voxel: A, or B at +axis (maybe in the next chunk)
+                    const uint32_t sx = x + (ax & air), sy = yl + (ay & air), sz = z + (az & air);
+                    const uint32_t at = ((sz & (R - 1)) << B | (sy & (R - 1))) << B | (sx & (R - 1));
+                    int16_t un = own_u;
+                    const uint8_t *p = own + at;
+                    if ((sx | sy | sz) & (uint32_t)R) {
+                        const int nbr = 13 + (sx >> B) + 3 * (sy >> B) + 9 * (sz >> B);
+                        un = s_uni[nbr];
+                        p = a.voxels + ((uint64_t)s_nid[nbr] << (3 * B)) + at;
                     }
-                    packed[k0 + u] = col[u] | shadow << 8 | diamond << 9 | ((w.meta >> 10) & 0x1FFu) << 11;
+                    cval[u] = un >= 0 ? (uint32_t)un : 0u;
+                    col[u] = 0u;
+                    if (un < 0) col[u] = *p;
+                    // Shadow samples (mesher.c:282-320, shadow.h:52-75), pairs of
+                    // neighbouring map entries: (i - 1, i) of the solid +x cell for
+                    // x faces of air; (i, i + 1) of the voxel for y faces of solid
+                    // voxels; for z faces (i, i + 1) of the cell in front and
+                    // (i - 1, i) one below it
+                    const uint32_t wx = ox + x;
+                    wy[u] = oy + yl;
+                    const uint32_t i = wx + wy[u] + ax + a.map_sx * (oz + z + (az & solid));
+                    const bool first = ax ? air != 0u : (ay ? solid != 0u : wy[u] != 0u);
+                    pair[u] = pair2[u] = 0u;
+                    if (first) __builtin_memcpy(&pair[u], a.map + (i - (ay ^ 1u)), 4);
+                    if (az) __builtin_memcpy(&pair2[u], a.map + i, 4);
                 }
-                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const uint32_t axis = e[u] & 3u, solid = e[u] >> 20, top = wy[u] + 1u;
+                    const uint32_t m1 = max(pair[u] & 0xFFFFu, pair[u] >> 16);
+                    const uint32_t m2 = max(pair2[u] & 0xFFFFu, pair2[u] >> 16);
+                    uint32_t shadow = 0, diamond = 3;
+                    if (axis == 2) {
+                        diamond = (m2 < top ? 2u : 0u) | (wy[u] != 0u && m1 < wy[u] ? 1u : 0u);
+                    } else if (axis == solid) {          // x faces of air, y faces of solid voxels
+                        shadow = m1 < top ? 0u : 1u;
+                    }
+                    const uint32_t code = axis + (solid ? 0u : 3u);
+                    const uint32_t j = j0 + (uint32_t)u * BS;
+                    if (j < pf)
+                        packed[j] = (col[u] | cval[u]) | code << 8 | shadow << 13 | diamond << 14 | amb[u] << 16;
+                }
+            };
+            for (uint32_t j0 = 0; j0 < pf;) {
+                const uint32_t left = (pf - j0 + BS - 1u) / BS;
+                if (left >= 3u) {
+                    prepare(std::integral_constant<int, 4>{}, j0 + threadIdx.x);
+                    j0 += 4u * BS;
+                } else {
+                    prepare(std::integral_constant<int, 1>{}, j0 + threadIdx.x);
+                    j0 += BS;
+                }
             }
-#pragma unroll
-            for (int kf = 0; kf < KF; kf++) {
-                const uint32_t j = threadIdx.x + (uint32_t)kf * BS;
-                if (j >= pf) break;
-                const uint32_t e = list[j];
-                const uint32_t axis = e & 3u, x = (e >> 2) & 63u, r = e >> 8;
-                const uint32_t z = r >> B, yl = r & (R - 1);
-                const uint32_t normal = ((uint32_t)(occ[(z + 1) * P + (yl + 1)] >> x) & 1u) ^ 1u;
-                const uint32_t pk = packed[kf];
-                const uint32_t common = (pk & 0xFFu) | (axis + 3u * normal) << 8 | ((pk >> 8) & 1u) << 13 |
-                                        ((pk >> 9) & 3u) << 14;
-                const uint32_t vao = (pk >> 11) & 0xFFu, rot = (pk >> 19) & 1u;
-                const uint32_t wx = ox + x, wy = oy + yl, wz = oz + z;
-                uint32_t wd[8];
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const uint32_t c = m_corner(axis, v);
-                    const uint32_t gx = (wx + (c & 1u)) & 0xFFFFu;
-                    const uint32_t gy = (wy + ((c >> 1) & 1u)) & 0xFFFFu;
-                    const uint32_t gz = (wz + (c >> 2)) & 0xFFFFu;
-                    const uint32_t attr = (common | ((vao >> (2 * v)) & 3u) << 6 | (uint32_t)v << 11) & 0xFFFFu;
-                    wd[2 * v] = gx | gy << 16;
-                    wd[2 * v + 1] = gz | attr << 16;
+            __syncthreads();
+            // E2: the stores, whole lines per instruction: half a face's vertices
+            // per lane, then a third of its indices
+            {
+                uint4 *gp = reinterpret_cast<uint4 *>(a.geom + 16 * (base + lo));
+                const uint32_t oxy = (ox & 0xFFFFu) | oy << 16;
+                for (uint32_t i = threadIdx.x; i < 2u * pf; i += BS) {
+                    const uint32_t e = list[i >> 1], pk = packed[i >> 1];
+                    const uint32_t x = (e >> 2) & 63u, r = (e >> 8) & 4095u;
+                    const uint4 c = s_corner[(e & 3u) << 1 | (i & 1u)];
+                    const uint32_t xy = oxy + (x | (r & (R - 1)) << 16);
+                    const uint32_t za = ((oz + (r >> B)) & 0xFFFFu) | pk << 16;
+                    const uint32_t amb = pk >> (16 + 4 * (i & 1u));
+                    nt_store16(gp + i, make_uint4(add_u16x2(xy, c.x),
+                                                  add_u16x2(za, c.y) | (amb & 3u) << 22,
+                                                  add_u16x2(xy, c.z),
+                                                  add_u16x2(za, c.w) | (amb & 12u) << 20));
                 }
-                const uint32_t fl = lo + j;                     // chunk-local face index
-                const uint64_t gf = base + fl;
-                uint4 *gp = reinterpret_cast<uint4 *>(a.geom + 16 * gf);
-                nt_store16(gp, make_uint4(wd[0], wd[1], wd[2], wd[3]));
-                nt_store16(gp + 1, make_uint4(wd[4], wd[5], wd[6], wd[7]));
-                const uint32_t vb = 4u * fl;
-                uint2 *ip = reinterpret_cast<uint2 *>(a.index + 6 * gf);
-                nt_store8(ip, make_uint2(vb + m_tri(normal, rot, 0), vb + m_tri(normal, rot, 1)));
-                nt_store8(ip + 1, make_uint2(vb + m_tri(normal, rot, 2), vb + m_tri(normal, rot, 3)));
-                nt_store8(ip + 2, make_uint2(vb + m_tri(normal, rot, 4), vb + m_tri(normal, rot, 5)));
-                __builtin_amdgcn_sched_barrier(0);   // one face at a time: bounded live ranges
+                uint2 *ip = reinterpret_cast<uint2 *>(a.index + 6 * (base + lo));
+                for (uint32_t i = threadIdx.x; i < 3u * pf; i += BS) {
+                    const uint32_t f = (i * 0xAAABu) >> 17, k = i - 3u * f;     // f = i / 3
+                    const uint32_t pk = packed[f];
+                    const uint32_t t = m_tri_row(((pk >> 8) & 7u) >= 3u, (pk >> 24) & 1u) >> (4u * k);
+                    const uint32_t vb = 4u * (lo + f);
+                    nt_store8(ip + i, make_uint2(vb + (t & 3u), vb + ((t >> 2) & 3u)));
+                }
             }
             __syncthreads();
             g0 = g1;
@@ -621,7 +648,7 @@ extern "C" int vp_gpu_mesh(vp_ctx *ctx, const vp_world_desc *world, const uint8_
     // 358 -> 131 us).
     const uint32_t resident = (uint32_t)ctx->num_cus * 2u;
     a.parts = 1u;
-    if (!count_only && n && n <= resident / 2u)
+    if (!count_only && root_bitw >= 5 && n && n <= resident / 2u)
         a.parts = std::min(1u << (root_bitw - 2u), resident / n);
     a.geom = count_only ? nullptr : out->d_geometry;
     a.index = count_only ? nullptr : out->d_index;

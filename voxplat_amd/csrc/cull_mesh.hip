@@ -691,6 +691,16 @@ __device__ __forceinline__ void emit_slices(const CullArgs &a, const ChunkRefs &
         nxt = take();
         fetch_win(nxt, wv);
         if (T == 0) continue;
+        // row y = R of level 0, written last: cells of the +y neighbour, lane x
+        // holds cell x; the colour's load overlaps the other rows' records
+        uint64_t rx = 0;
+        uint32_t ycol = 0;
+        if (l == 0) {
+            rx = uni(lds[L::V0 + s * N0 + R]);
+            if ((rx >> ln) & 1ull)
+                ycol = c.nb_u[1] >= 0 ? (uint32_t)c.nb_u[1]
+                                      : (uint32_t)c.nb[1][(size_t)s * R * R + ln];
+        }
         const uint64_t *rows = l == 0 ? lds + L::V0 + s * N0
                                       : lds + L::P1 + (G::row_base(l) - G::RB1) + s * nl;
         const int lanes = l == 0 ? R : nl;             // row y = R of level 0 comes last
@@ -805,14 +815,10 @@ __device__ __forceinline__ void emit_slices(const CullArgs &a, const ChunkRefs &
             b0 = b1;
         }
         if (l == 0 && tot < T) {
-            // row y = R: cells of the +y neighbour, lane x holds cell x
-            const uint64_t rx = uni(rows[R]);
             if ((rx >> ln) & 1ull) {
-                const uint32_t col = c.nb_u[1] >= 0 ? (uint32_t)c.nb_u[1]
-                                                    : (uint32_t)c.nb[1][(size_t)s * R * R + ln];
                 const bool sh = win[ln + R] > R;
                 const uint32_t lo = base + ln + ((uint32_t)R << 16);
-                const uint32_t hi = wz | col << 16 |
+                const uint32_t hi = wz | ycol << 16 |
                                     (V2 ? 8u << 24 | (sh ? 1u << 30 : 0u) : (sh ? 1u << 22 : 0u));
                 __builtin_nontemporal_store((uint64_t)hi << 32 | lo, o + tot + rank_below(rx));
             }
@@ -1170,13 +1176,14 @@ __device__ __forceinline__ void cull_chunk(const CullArgs &a, uint32_t k, uint32
 // z-slices are independent ranges of the output, so the parts repeat the cull
 // and count (reads that the caches serve) and share the slices out: one 64^3
 // chunk 47.3 -> 28.9 us, the 32 chunks of a few edits 178 -> 45-48 us.  At most
-// R / 4 of them: the slices left to a part then cost less than its cull.
+// R / 4 of them: the slices left to a part then cost less than its cull.  Chunks
+// below 32^3 are too small to gain (64 of 16^3: 31 us whole, 36 us in parts).
 template <int B>
-constexpr uint32_t max_parts() { return B < 2 ? 1u : 1u << (B - 2); }
+constexpr uint32_t max_parts() { return B < 5 ? 1u : 1u << (B - 2); }
 
 static uint32_t max_parts_of(uint32_t root_bitw, bool count_only)
 {
-    return count_only || root_bitw < 2 ? 1u : 1u << (root_bitw - 2);
+    return count_only || root_bitw < 5 ? 1u : 1u << (root_bitw - 2);
 }
 
 // LDS (about 67 KiB at 512 threads for R = 64) allows two workgroups per CU;
@@ -1340,7 +1347,17 @@ int cull_mesh_launch(vp_ctx *ctx, const vp_world_desc *world, const uint8_t *d_v
     a.level_counts = out->d_level_counts;
     a.status = ctx->d_status;
     a.nchunks = (uint32_t)(1ull << (world->max_bitw[0] + world->max_bitw[1] + world->max_bitw[2]));
-    const vp_remesh_shape_i sh = remesh_shape(ctx, world);
+    vp_remesh_shape_i sh = remesh_shape(ctx, world);
+    // Where nobody chose a shape, 64^3 chunks are emitted by one 1024-thread
+    // workgroup per CU: it has the LDS for the coarser levels' colours (all
+    // chunks of 2048x256x2048 at 512 threads: 1246 us, at 1024: 962; 512 chunks
+    // 260, 160).  With face flags two records in flight are the faster (1024
+    // chunks: 659 us at 512 threads, 459 with four, 435 with two).
+    if (!sh.chosen && world->root_bitw == 6 && !a.count_only) {
+        sh.block = 1024;
+        sh.wg_per_cu = 1;
+        sh.u = (flags & VP_CM_RECORD_V2) ? 2 : 4;
+    }
     const uint32_t parts = max_parts_of(world->root_bitw, a.count_only != 0);
     int grid = a.single ? (int)parts : 1, bs = sh.block;
     // one 64^3 chunk alone: a 1024-thread workgroup (16 waves on one CU)

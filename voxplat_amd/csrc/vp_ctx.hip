@@ -240,6 +240,7 @@ extern "C" int vp_ctx_set_launch(vp_ctx *ctx, int block, int wg_per_cu)
     std::lock_guard<std::mutex> g(ctx->mu);
     ctx->cull_shape.block = block;
     ctx->cull_shape.wg_per_cu = wg_per_cu;
+    ctx->cull_shape.chosen = true;
     return VP_OK;
 }
 
@@ -263,6 +264,7 @@ extern "C" int vp_ctx_set_remesh_shape(vp_ctx *ctx, const vp_world_desc *world,
     s.block = b;
     s.wg_per_cu = w;
     s.u = u;
+    s.chosen = true;
     std::lock_guard<std::mutex> g(ctx->mu);
     if (!world) {
         ctx->cull_shape = s;

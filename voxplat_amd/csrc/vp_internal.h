@@ -20,6 +20,7 @@ struct vp_remesh_shape_i {
     int block = 512;
     int wg_per_cu = 2;
     int u = 4;
+    bool chosen = false;    // set by the caller or the autotuner
 };
 
 struct vp_ctx {

@@ -650,22 +650,28 @@ __device__ __forceinline__ void emit_slices(const CullArgs &a, const ChunkRefs &
     auto write = [&](uint64_t *ob, uint32_t nb, auto &&load, auto &&make) {
         const __amdgpu_buffer_rsrc_t ro = byte_rsrc(ob, nb * 8u);
         const uint32_t jmax = nb - 1u;
-#pragma unroll 1
-        for (uint32_t j0 = 0; j0 < nb; j0 += 64 * U) {
-            uint32_t e[U], col[U];
+        auto some = [&](auto uc, uint32_t j0) {
+            constexpr int N = decltype(uc)::value;
+            uint32_t e[N], col[N];
 #pragma unroll
-            for (int u = 0; u < U; u++) {
+            for (int u = 0; u < N; u++) {
                 const uint32_t j = j0 + (uint32_t)u * 64u + ln;
                 e[u] = list[min(j, jmax)];
                 col[u] = load(e[u]);
             }
 #pragma unroll
-            for (int u = 0; u < U; u++) {
+            for (int u = 0; u < N; u++) {
                 uint32_t lo, hi;
                 make(e[u], col[u], lo, hi);
                 st8_nt(ro, (j0 + (uint32_t)u * 64u + ln) * 8u, lo, hi);
             }
-        }
+        };
+        // a wave pays for every record slot, also past the batch: short rests
+        // (most slices of small chunks' coarser levels) take one at a time
+        uint32_t j0 = 0;
+#pragma unroll 1
+        for (; j0 + 64u < nb; j0 += 64 * U) some(std::integral_constant<int, U>{}, j0);
+        if (j0 < nb) some(std::integral_constant<int, 1>{}, j0);
     };
     uint32_t nxt = take();
     uint32_t wv[WQ];

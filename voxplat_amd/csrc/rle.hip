@@ -61,11 +61,13 @@ __device__ __forceinline__ uint32_t diff4(uint32_t w, uint32_t prev)
 template <int B, int BS>
 struct EncodeLds {
     static constexpr int VOX = 1 << (3 * B), WORDS = VOX / 64, NG = (WORDS + 63) / 64;
-    static constexpr int CAP = VOX < 2048 ? VOX : 2048;     // starts a wave lists at a time
+    static constexpr int CAP = VOX < 960 ? VOX : 960;       // starts a wave lists at a time
+    static constexpr int GB = VOX < 4096 ? VOX : 4096;      // bytes of a group of 64 words
     uint64_t bm[WORDS];             // bit per voxel: a run starts here
     uint32_t gtot[NG], gfirst[NG];  // per 64 bitmap words: starts, and the first of them
     uint64_t base;
     uint32_t ticket;
+    uint4    vox[BS / 64][(GB + 15) / 16];
     uint16_t list[BS / 64][CAP];
 };
 
@@ -90,8 +92,8 @@ __device__ void rle_encode_chunk(const RleArgs &a, uint32_t k, uint32_t n, Encod
     // A chunk the caller's uniform table marks uniform (every voxel holds that
     // value; edits mark their chunks mixed) is one run and the terminator:
     // none of its voxels is read.
-    const int uval = (src && a.uniform_in) ? (int)a.uniform_in[chunk] : -1;
-    const bool fast = uval >= 0;
+    int uval = (src && a.uniform_in) ? (int)a.uniform_in[chunk] : -1;
+    bool fast = uval >= 0;
     uint32_t runs = 1, gbeg = 0, gnext = 0;
     constexpr int NW = BS / 64, NG = EncodeLds<B, BS>::NG;
     const uint32_t ln = r_lane();
@@ -164,6 +166,24 @@ __device__ void rle_encode_chunk(const RleArgs &a, uint32_t k, uint32_t n, Encod
     }
     }   // !fast
 
+    if (runs == 1u && !fast) {          // one value after all
+        uval = src ? (int)src[0] : 0;
+        fast = true;
+    }
+    // the voxels of a wave's first group are on their way during the look-back
+    constexpr int GQ = (EncodeLds<B, BS>::GB / 16 + 63) / 64;
+    uint4 ahead[GQ];
+    auto fetch = [&](int g) {
+#pragma unroll
+        for (int q = 0; q < GQ; q++) {
+            const int i = (int)ln + 64 * q;
+            ahead[q] = make_uint4(0u, 0u, 0u, 0u);
+            if (src && g < NG && i * 16 < EncodeLds<B, BS>::GB)
+                ahead[q] = *reinterpret_cast<const uint4 *>(src + (size_t)g * 4096 + (size_t)i * 16);
+        }
+    };
+    if (!fast && a.words) fetch(wv);
+
     // ---- 3. publish the word count (runs + terminator), look back ----
     const uint64_t nwords = (uint64_t)runs + 1u;
     if (threadIdx.x < 64) {
@@ -201,8 +221,7 @@ __device__ void rle_encode_chunk(const RleArgs &a, uint32_t k, uint32_t n, Encod
             a.offsets[k] = excl;
             if (k + 1 == n) a.offsets[n] = excl + nwords;
             if (a.uniform_out)
-                a.uniform_out[k] = fast ? (int16_t)uval
-                                 : (runs == 1) ? (int16_t)(src ? src[0] : 0) : (int16_t)-1;
+                a.uniform_out[k] = fast ? (int16_t)uval : (int16_t)-1;
             if (a.words && excl + nwords > a.cap) atomicOr(a.status, (uint32_t)VP_STATUS_OVERFLOW);
         }
     }
@@ -213,8 +232,8 @@ __device__ void rle_encode_chunk(const RleArgs &a, uint32_t k, uint32_t n, Encod
     // ---- 4. words ----
     // A wave takes a group of 64 bitmap words at a time: each lane lists its
     // word's starts in LDS, then consecutive lanes take consecutive runs, so
-    // that the values' loads fall in few lines and the words' stores are whole
-    // lines (a lane per bitmap word instead, 64 lines for each: 1.6x the time).
+    // that the words' stores are whole lines.  The group's voxels come through
+    // LDS, loaded a group ahead.
     // A group with more starts than the list holds goes in batches of words.
     uint32_t *out = a.words + base;
     if (fast) {
@@ -229,7 +248,12 @@ __device__ void rle_encode_chunk(const RleArgs &a, uint32_t k, uint32_t n, Encod
             uint32_t tot;
             const uint32_t off = wave_excl_scan(cnt, tot);
             uint32_t *og = out + (uint32_t)__builtin_amdgcn_readlane((int)gbeg, g);
-            const uint8_t *sg = src + (size_t)g * 4096;
+            const uint8_t *sg = reinterpret_cast<const uint8_t *>(L.vox[wv]);
+            wave_order();                      // the previous group's reads are done
+#pragma unroll
+            for (int q = 0; q < GQ; q++)
+                if (((int)ln + 64 * q) * 16 < EncodeLds<B, BS>::GB) L.vox[wv][(int)ln + 64 * q] = ahead[q];
+            fetch(g + NW);
             const uint32_t gend = (uint32_t)__builtin_amdgcn_readlane((int)gnext, g) - (uint32_t)g * 4096u;
 #pragma unroll 1
             for (uint32_t b0 = 0; b0 < tot;) {
@@ -265,7 +289,7 @@ __device__ void rle_encode_chunk(const RleArgs &a, uint32_t k, uint32_t n, Encod
                         const uint32_t j = min(j0 + (uint32_t)u * 64u + ln, nb - 1u);
                         pos[u] = list[j];
                         end[u] = j + 1u < nb ? (uint32_t)list[j + 1u] : after;
-                        val[u] = src ? (uint32_t)sg[pos[u]] : 0u;
+                        val[u] = (uint32_t)sg[pos[u]];
                     }
 #pragma unroll
                     for (int u = 0; u < U; u++) {

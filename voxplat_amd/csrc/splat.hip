@@ -874,8 +874,8 @@ __global__ void __launch_bounds__(kBlock) k_raster_blocks(const int16_t *splats,
     flush(0u, lane < held);
 }
 
-// The visible blocks without the tile bounds (frames of up to kFewPixels): a
-// workgroup per block, a splat per thread.
+// The visible blocks without the tile bounds (frames of up to kFewPixels, and
+// cameras that bounds_hold rules out): a workgroup per block, a splat per thread.
 __global__ void __launch_bounds__(kBlock) k_raster_few(const int16_t *splats, const uint8_t *lod,
                                                         uint32_t lod_log2, uint64_t n, SplatCam c,
                                                         const float4 *rays, uint64_t *frame,
@@ -1433,6 +1433,61 @@ static CullPlanes cull_planes(const vp_camera *cam)
     return cp;
 }
 
+// Whether the tile bounds' approximate arithmetic (splat_open, block_box) stays
+// within its margins for this camera.  It does for a view translation followed
+// by a perspective projection of a rotated view, the camera vp_camera names:
+//  * a translation gives the view position one rounding, fl(a + t), however it
+//    is summed, so both sides start from the same position v; any other matrix
+//    rounds at the size of the world's coordinates, not of v, and splats near
+//    the eye would be judged by an error of their own size;
+//  * clip coordinates are sums of four products, at most 8 half-ulps apart on
+//    the two sides: g = 8 2^-24 times a row's absolute sum, times |v|.  A splat
+//    in the volume has |clip x|, |clip y| <= w, so |v| <= L w (+ a constant),
+//    L from the inverse of the rows x, y and w;
+//  * the third row follows the fourth, so clip z, which sizes the sprites, is
+//    no smaller than half of w beside its own constant.
+// 2 g L must stay below splat_open's 1e-4 of w, and its share of a pixel, g L
+// times the wider side, below 0.2 of its margin of 0.25.
+static bool bounds_hold(const vp_camera *cam)
+{
+    const float *T = cam->view_translation, *P = cam->proj_view_rot;
+    for (int k = 0; k < 3; k++)
+        for (int r = 0; r < 4; r++)
+            if (T[4 * k + r] != (r == k ? 1.0f : 0.0f)) return false;
+    if (T[15] != 1.0f || !(cam->far_plane > 1e-30f && cam->far_plane < 1e30f)) return false;
+    const double ulps = 8.0 / 16777216.0;
+    double sum = 0.0, con = 0.0, A[3][3];          // A: rows x, y, w
+    for (int r = 0; r < 4; r++) {
+        double s = 0.0;
+        for (int k = 0; k < 3; k++) s += fabs((double)P[4 * k + r]);
+        sum = fmax(sum, s);
+        con = fmax(con, fabs((double)P[12 + r]));
+        for (int k = 0; k < 3 && r != 2; k++) A[r == 3 ? 2 : r][k] = P[4 * k + r];
+    }
+    auto cof = [&](int r, int k) {
+        const int r1 = (r + 1) % 3, r2 = (r + 2) % 3, k1 = (k + 1) % 3, k2 = (k + 2) % 3;
+        return A[r1][k1] * A[r2][k2] - A[r1][k2] * A[r2][k1];
+    };
+    const double det = A[0][0] * cof(0, 0) + A[0][1] * cof(0, 1) + A[0][2] * cof(0, 2);
+    double L = 0.0, zz = 0.0, zw = 0.0;
+    for (int k = 0; k < 3; k++) {
+        double s = 0.0;
+        for (int r = 0; r < 3; r++) s += fabs(cof(r, k));
+        L = fmax(L, s / fabs(det));
+        zw += (double)P[4 * k + 2] * A[2][k];
+        zz += A[2][k] * A[2][k];
+    }
+    const double scale = zw / zz;                  // the third row in the fourth's
+    for (int k = 0; k < 3; k++)
+        if (!(fabs(P[4 * k + 2] - scale * A[2][k]) <= 1e-5 * sqrt(zz))) return false;
+    // |v| <= L (w + |constant|): the constants of x, y and w count as w's
+    for (int r = 0; r < 4; r++)
+        if (r != 2 && !(fabs(P[12 + r]) <= 1.0f)) return false;
+    const double e = ulps * sum * L, e0 = e + ulps * con, side = fmax(cam->width, cam->height);
+    return scale >= 0.5 && con <= 100.0 && 2.0 * e <= 1e-4 && 2.0 * e0 <= 1e-3 &&
+           (e + 0.5 * e0) * side <= 0.2 && sum < 1e6;
+}
+
 // The splat frame.  d_n (nullable): the list length in device memory, n its
 // bound; with d_n the block bounds are computed into d_bounds here first (the
 // list is assembled on the device each frame).
@@ -1520,7 +1575,7 @@ static int splat_frame(vp_ctx *ctx, const int16_t *d_splats, const uint8_t *d_lo
         const float reach = (float)c.H * 1.1f * (float)(1u << lod_log2) / kNearPixels;
         const uint32_t near_bin =
             (uint32_t)fminf(fmaxf(sqrtf(reach / c.far_plane) * (float)kBins, 0.0f), (float)kBins);
-        const bool few = np <= kFewPixels;
+        const bool few = np <= kFewPixels || !bounds_hold(cam);
         const uint32_t g = (uint32_t)((nb + 255) / 256 < 4096 ? (nb + 255) / 256 : 4096);
         hipLaunchKernelGGL(k_blk_cull, dim3(g), dim3(256), 0, st, d_bounds, nb, cull_planes(cam),
                            c, bin, few ? nullptr : box, cnt, d_n);

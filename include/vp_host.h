@@ -26,9 +26,13 @@ int vp_ctx_reserve(vp_ctx *ctx, uint64_t max_chunks, uint64_t max_pixels);
  * records each lane prepares before it stores them (2 or 4; chunks of 64^3
  * only, smaller chunks always use 4).  No counterpart in the reference, which
  * meshes on the CPU.  A world without a shape of its own (set for its
- * root_bitw and max_bitw) uses the default (world = NULL): 512, 2, 4.  Until
- * a default or a world's shape is set, lists of 64^3 chunks that write records
- * run 1024 threads, one workgroup per CU, whatever the default says. */
+ * root_bitw and max_bitw) uses the default (world = NULL).  Until one is set,
+ * lists that write records run 1024, 1, 4 for chunks of 64^3 (2 records in
+ * flight with face flags) and 512, 2, 4 below; sizing passes run 512, 2, 4.
+ * The getter answers the shape such a list runs (world = NULL: of 64^3 chunks,
+ * 1024, 1, 4 where none is set), and setting those values is the unset state
+ * again: read, set another, put back.  (1024, 1, 4 as the default therefore
+ * leaves smaller chunks at 512, 2, 4; set it for their world to run it.) */
 typedef struct {
     int block;
     int wg_per_cu;
@@ -42,7 +46,7 @@ int vp_ctx_get_remesh_shape(vp_ctx *ctx, const vp_world_desc *world, vp_remesh_s
  * wg_per_cu above it only queues workgroups. */
 int vp_ctx_remesh_resident(vp_ctx *ctx, const vp_world_desc *world, uint32_t flags,
                            const vp_remesh_shape *shape, int *per_cu);
-/* The default shape's block and wg_per_cu. */
+/* The default shape's block and wg_per_cu (1024, 1 where none is set). */
 int vp_ctx_set_launch(vp_ctx *ctx, int block, int wg_per_cu);
 int vp_ctx_get_launch(vp_ctx *ctx, int *block, int *wg_per_cu);
 

@@ -1353,17 +1353,18 @@ int cull_mesh_launch(vp_ctx *ctx, const vp_world_desc *world, const uint8_t *d_v
     a.level_counts = out->d_level_counts;
     a.status = ctx->d_status;
     a.nchunks = (uint32_t)(1ull << (world->max_bitw[0] + world->max_bitw[1] + world->max_bitw[2]));
-    vp_remesh_shape_i sh = remesh_shape(ctx, world);
     // Where nobody chose a shape, 64^3 chunks are emitted by one 1024-thread
     // workgroup per CU: it has the LDS for the coarser levels' colours (all
     // chunks of 2048x256x2048 at 512 threads: 1246 us, at 1024: 962; 512 chunks
     // 260, 160).  With face flags two records in flight are the faster (1024
-    // chunks: 659 us at 512 threads, 459 with four, 435 with two).
-    if (!sh.chosen && world->root_bitw == 6 && !a.count_only) {
-        sh.block = 1024;
-        sh.wg_per_cu = 1;
-        sh.u = (flags & VP_CM_RECORD_V2) ? 2 : 4;
-    }
+    // chunks: 659 us at 512 threads, 459 with four, 435 with two).  Sizing
+    // passes keep two workgroups of 512 threads.
+    bool unset;
+    vp_remesh_shape_i sh = remesh_shape(ctx, world, unset);
+    if (unset && a.count_only)
+        sh = {512, 2, 4};
+    else if (unset && world->root_bitw == 6 && (flags & VP_CM_RECORD_V2))
+        sh.u = 2;
     const uint32_t parts = max_parts_of(world->root_bitw, a.count_only != 0);
     int grid = a.single ? (int)parts : 1, bs = sh.block;
     // one 64^3 chunk alone: a 1024-thread workgroup (16 waves on one CU)

@@ -240,7 +240,6 @@ extern "C" int vp_ctx_set_launch(vp_ctx *ctx, int block, int wg_per_cu)
     std::lock_guard<std::mutex> g(ctx->mu);
     ctx->cull_shape.block = block;
     ctx->cull_shape.wg_per_cu = wg_per_cu;
-    ctx->cull_shape.chosen = true;
     return VP_OK;
 }
 
@@ -260,11 +259,7 @@ extern "C" int vp_ctx_set_remesh_shape(vp_ctx *ctx, const vp_world_desc *world,
     const int b = shape->block, w = shape->wg_per_cu, u = shape->records_in_flight;
     if ((b != 256 && b != 512 && b != 1024) || w < 1 || w > 4 || (u != 2 && u != 4))
         return VP_ERR_ARG;
-    vp_remesh_shape_i s;
-    s.block = b;
-    s.wg_per_cu = w;
-    s.u = u;
-    s.chosen = true;
+    const vp_remesh_shape_i s = {b, w, u};
     std::lock_guard<std::mutex> g(ctx->mu);
     if (!world) {
         ctx->cull_shape = s;
@@ -287,7 +282,8 @@ extern "C" int vp_ctx_get_remesh_shape(vp_ctx *ctx, const vp_world_desc *world,
 {
     if (!ctx || !shape) return VP_ERR_ARG;
     std::lock_guard<std::mutex> g(ctx->mu);
-    const vp_remesh_shape_i s = world ? vp::remesh_shape(ctx, world) : ctx->cull_shape;
+    bool unset;
+    const vp_remesh_shape_i s = world ? vp::remesh_shape(ctx, world, unset) : ctx->cull_shape;
     shape->block = s.block;
     shape->wg_per_cu = s.wg_per_cu;
     shape->records_in_flight = s.u;

@@ -17,11 +17,24 @@
 // workgroups per CU the grid is sized for, records each lane prepares
 // before its stores.
 struct vp_remesh_shape_i {
-    int block = 512;
-    int wg_per_cu = 2;
-    int u = 4;
-    bool chosen = false;    // set by the caller or the autotuner
+    int block;
+    int wg_per_cu;
+    int u;
 };
+
+inline bool operator==(const vp_remesh_shape_i &a, const vp_remesh_shape_i &b)
+{
+    return a.block == b.block && a.wg_per_cu == b.wg_per_cu && a.u == b.u;
+}
+
+// The shape of lists that write records where none was chosen: 64^3 chunks run
+// one 1024-thread workgroup per CU, smaller ones 512 threads, two per CU.  A
+// shape set to these values is this state again, so that a caller who reads the
+// shape, sets another and puts the first back is where it began.
+inline vp_remesh_shape_i unset_shape(uint32_t root_bitw)
+{
+    return root_bitw == 6 ? vp_remesh_shape_i{1024, 1, 4} : vp_remesh_shape_i{512, 2, 4};
+}
 
 struct vp_ctx {
     int device = 0;
@@ -54,8 +67,10 @@ struct vp_ctx {
     // this context's device (noalloc.hip); not owned
     uint64_t *d_noalloc = nullptr;
     // launch shape of the persistent remesh kernel: a default, and tuned
-    // shapes per world geometry (key: root_bitw | max_bitw[a] << 8 (a + 1))
-    vp_remesh_shape_i cull_shape;
+    // shapes per world geometry (key: root_bitw | max_bitw[a] << 8 (a + 1)).
+    // The default stands for every chunk edge and is unset where it equals the
+    // 64^3 chunks' shape; a world's own is unset where it equals its edge's.
+    vp_remesh_shape_i cull_shape = unset_shape(6);
     static constexpr int kMaxShapes = 16;
     uint32_t cull_shape_key[kMaxShapes] = {};
     vp_remesh_shape_i cull_shapes[kMaxShapes];
@@ -81,15 +96,22 @@ inline uint32_t world_key(const vp_world_desc *w)
            (uint32_t)w->max_bitw[2] << 24;
 }
 
-// The remesh launch shape for a world: its tuned shape, else the default.
+// The remesh launch shape for a world: its tuned shape, else the default, else
+// the one of its chunk edge.  unset: whether it is the last (of lists that
+// write records; the launch has its own for sizing passes and face flags).
 // Read without the context lock (launches may hold it); shapes are set
 // between calls, not during them.
-inline vp_remesh_shape_i remesh_shape(const vp_ctx *ctx, const vp_world_desc *w)
+inline vp_remesh_shape_i remesh_shape(const vp_ctx *ctx, const vp_world_desc *w, bool &unset)
 {
     const uint32_t k = world_key(w);
+    vp_remesh_shape_i s = ctx->cull_shape;
+    unset = s == unset_shape(6);
     for (int i = 0; i < ctx->n_cull_shapes; i++)
-        if (ctx->cull_shape_key[i] == k) return ctx->cull_shapes[i];
-    return ctx->cull_shape;
+        if (ctx->cull_shape_key[i] == k) {
+            s = ctx->cull_shapes[i];
+            unset = s == unset_shape(w->root_bitw);
+        }
+    return unset ? unset_shape(w->root_bitw) : s;
 }
 
 // vp_gpu_cull_mesh's argument checks, and its launch with explicit scratch:

@@ -224,14 +224,18 @@ __device__ __forceinline__ void fragment_test(const SplatCam &c, float4 inv, uin
 // larger ones by the whole wave, a few at a time.  Most fragments end at
 // the depth lower bound after one frame load, so the loads are issued in
 // batches (kLoads per lane) before any test: the lane waits once per batch
-// instead of once per pixel.  Batches of 4: a slot costs its instructions
-// whether a lane has a pixel for it or not, and a splat covers 6 pixels on
-// average (8: 913 against 881 us per 1080p frame, 4776 against 4426 us for 16
-// views of 512x512; 2: 975 us; 12 leaves three waves per SIMD: 1367 us).
+// instead of once per pixel.  A lane's own sprite takes batches of 4: a slot
+// costs its instructions whether a lane has a pixel for it or not, and a splat
+// covers 6 pixels on average (8: 913 against 881 us per 1080p frame, 4776
+// against 4426 us for 16 views of 512x512; 2: 975 us; 12 leaves three waves per
+// SIMD: 1367 us).  Wave-shared sprites fill their slots, and take 8 (two close
+// views of a 7.7 M list at 1697x1495: 8030 us with 4, 5810 with 8; of a 31 M
+// list at 1920x1080: 5760, 4440).
 constexpr int kSmallArea = 64;
 constexpr int kLoads = 4;
-constexpr int kGroup = 2;                 // wave-shared sprites per round
-constexpr int kSteps = kLoads / kGroup;   // pixels of each per lane per round
+constexpr int kGroup = 4;                 // wave-shared sprites per round
+constexpr int kSteps = 2;                 // pixels of each per lane per round
+constexpr int kShared = kGroup * kSteps;
 
 // Lane src's value (src wave-uniform) through a scalar register: no LDS
 // traffic, unlike a general shuffle.
@@ -330,8 +334,8 @@ __device__ __forceinline__ void raster_splat(bool ok, uint2 rec, float lodf, uin
             }
         }
         for (int k0 = 0; k0 < amax; k0 += 64 * kSteps) {
-            uint32_t pp[kLoads];
-            uint64_t cur[kLoads];
+            uint32_t pp[kShared];
+            uint64_t cur[kShared];
             uint32_t live = 0;
 #pragma unroll
             for (int g = 0; g < kGroup; g++)

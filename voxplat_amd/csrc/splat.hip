@@ -267,7 +267,12 @@ __device__ __forceinline__ WaveSprite wave_sprite(const VS &vs, int area, uint32
 }
 
 // One splat per lane (ok: the lane has one), record rec of edge lodf; every
-// lane of the wave calls it.
+// lane of the wave calls it.  AHEAD: a batch's rays are loaded together before
+// its tests.  Near to far, few fragments pass the bound and their rays' waits
+// add up; in list order many pass, and the loads beside those that do not cost
+// more than the waits (a 7.7 M list at 1920x1080 without blocks, four far views:
+// 5220 us ahead, 4900 on demand).
+template <bool AHEAD>
 __device__ __forceinline__ void raster_splat(bool ok, uint2 rec, float lodf, uint32_t id,
                                              const SplatCam &c, const float4 *rays,
                                              uint64_t *frame)
@@ -294,15 +299,16 @@ __device__ __forceinline__ void raster_splat(bool ok, uint2 rec, float lodf, uin
                 p += last ? turn : 1u;
                 end += last ? c.W : 0u;
             }
-            // the rays of the pixels that pass the bound, together
+            // AHEAD: the rays of the pixels that pass the bound, together
 #pragma unroll
             for (int u = 0; u < kLoads; u++) {
                 inv[u] = make_float4(1.0f, 1.0f, 1.0f, 0.0f);
-                if (vs.lb <= cur[u]) inv[u] = rays[pp[u]];
+                if (AHEAD && vs.lb <= cur[u]) inv[u] = rays[pp[u]];
             }
 #pragma unroll
             for (int u = 0; u < kLoads; u++)
-                if (vs.lb <= cur[u]) fragment_test(c, inv[u], frame, sl, id, pp[u], cur[u]);
+                if (vs.lb <= cur[u])
+                    fragment_test(c, AHEAD ? inv[u] : rays[pp[u]], frame, sl, id, pp[u], cur[u]);
         }
     }
     uint64_t big = __ballot(area > kSmallArea);
@@ -376,7 +382,7 @@ __device__ __forceinline__ void raster_list(const int16_t *splats, const uint8_t
         rec = ld_rec(splats, i);
         lodf = (float)(1u << (lod ? lod[i] : lod_log2));
     }
-    raster_splat(i < n, rec, lodf, (uint32_t)i, c, rays, frame);
+    raster_splat<false>(i < n, rec, lodf, (uint32_t)i, c, rays, frame);
 }
 
 // One thread per splat, in list order.
@@ -807,7 +813,7 @@ __global__ void __launch_bounds__(kBlock) k_raster_blocks(const int16_t *splats,
     auto flush = [&](uint32_t at, bool ok) {
         const uint32_t e = at + lane;
         const uint2 rec = ok ? make_uint2(q.x[e], q.y[e]) : make_uint2(0u, 0u);
-        raster_splat(ok, rec, ok ? (float)(1u << q.lv[e]) : 1.0f, ok ? q.id[e] : 0u, c, rays, frame);
+        raster_splat<true>(ok, rec, ok ? (float)(1u << q.lv[e]) : 1.0f, ok ? q.id[e] : 0u, c, rays, frame);
     };
     // units of work: the quarters of the near blocks, then whole blocks
     const uint32_t near = cnt[kNear], units = total + 3u * near;
@@ -898,7 +904,7 @@ __global__ void __launch_bounds__(kBlock) k_raster_few(const int16_t *splats, co
             rec = *reinterpret_cast<const uint2 *>(splats + 4 * i);
             if (lod) lv = lod[i];
         }
-        raster_splat(i < n, rec, (float)(1u << lv), (uint32_t)i, c, rays, frame);
+        raster_splat<true>(i < n, rec, (float)(1u << lv), (uint32_t)i, c, rays, frame);
     }
 }
 

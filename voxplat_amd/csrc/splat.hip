@@ -767,13 +767,20 @@ constexpr float kNearPixels = 5.0f;
 // 421 us, 489x499 of 114 M: 524 against 552 us; 757x591: 489 against 498 us, and
 // 928x743 of 3.3 M: 152 against 131 us).
 constexpr uint64_t kFewPixels = 1u << 18;
+// Tile groups (4 KiB of keys each) a wave refreshes at a time.  Its whole share
+// is up to 4 groups on 256 CUs at 3840x2160 and 128 at 16384x16384, where reading
+// all of it every second block cost more than the bounds saved (four far views of
+// a 31 M list 207.6 ms; 4 at a time 165.2; without the bounds 175; one at a time
+// 2422x2321 takes 5430 against 5060 us).
+constexpr uint32_t kRefresh = 4;
 constexpr uint32_t kHeld = kBlock + 64;   // a wave's queue: less than a wave, and a block
 // Wave w takes the ordered blocks w, w + G, w + 2G, ... (G waves): every wave
 // starts at the near end of the order, no counter is shared, and the waves
 // never wait for each other.  A block that is hidden is skipped; of the others
 // the splats that may still win a pixel go to the wave's queue in LDS, and
-// full waves of them are rasterised.  Every second block a wave refreshes its
-// share of the tile bounds (every block or every fourth: within 3%).
+// full waves of them are rasterised.  Every second block a wave refreshes up to
+// kRefresh groups of its share of the tile bounds, in turn (every block or every
+// fourth: within 3%).
 // Bound by vector instructions (78% of the SIMDs' issue slots): a 1920x1080
 // frame of a 130.5 M list has 312 K blocks and 77 M splats in view, of which
 // 48% and 20% are not dropped here; each splat rasterised costs some hundred
@@ -809,7 +816,7 @@ __global__ void __launch_bounds__(kBlock) k_raster_blocks(const int16_t *splats,
     const uint32_t share = (nt + nw - 1) / nw;
     const uint32_t h0 = min(w * share, nt), h1 = min(h0 + share, nt);
     constexpr int PER = kBlock / 64;
-    uint32_t held = 0, turn = 0;
+    uint32_t held = 0, turn = 0, hg = h0;
     auto flush = [&](uint32_t at, bool ok) {
         const uint32_t e = at + lane;
         const uint2 rec = ok ? make_uint2(q.x[e], q.y[e]) : make_uint2(0u, 0u);
@@ -879,7 +886,11 @@ __global__ void __launch_bounds__(kBlock) k_raster_blocks(const int16_t *splats,
             flush(held, true);
         }
         wave_fence();
-        if (++turn & 1u) hiz_refresh(frame, hiz, c.W, c.H, h0, h1);
+        if (++turn & 1u) {
+            const uint32_t he = min(hg + kRefresh, h1);
+            hiz_refresh(frame, hiz, c.W, c.H, hg, he);
+            hg = he < h1 ? he : h0;
+        }
     }
     flush(0u, lane < held);
 }

@@ -114,7 +114,7 @@ struct Lay : Rows<B, V2> {
     {
         return l <= 1 ? 0 : cbase(l - 1) + cube(Geo<B>::n(l - 1));
     }
-    // per wave: LCAP list entries and SWIN shadow entries.  An entry is the
+    // per wave: LCAP list entries and SWIN shadow bytes.  An entry is the
     // cell code y << 7 | x, u16 in the MIP kernel (which keeps no level-1
     // child selection in it, so its lists hold 1920 cells: most slices in
     // one batch, and the byte plane below still fits), else u32 with the
@@ -1181,7 +1181,7 @@ __device__ __forceinline__ void cull_chunk(const CullArgs &a, uint32_t k, uint32
 // A 64^3 chunk's workgroup spends most of its time on the emission, whose
 // z-slices are independent ranges of the output, so the parts repeat the cull
 // and count (reads that the caches serve) and share the slices out: one 64^3
-// chunk 47.3 -> 28.9 us, the 32 chunks of a few edits 178 -> 45-48 us.  At most
+// chunk 47.3 -> 28.9 us, the 32 chunks of a few edits 171 -> 41 us.  At most
 // R / 4 of them: the slices left to a part then cost less than its cull.  Chunks
 // below 32^3 are too small to gain (64 of 16^3: 31 us whole, 36 us in parts).
 template <int B>

@@ -7,11 +7,11 @@
 //
 // One workgroup per chunk (persistent, ticket order = list order):
 //  1. the chunk's occupancy and a one-voxel shell around it, (R+2)^3 bits,
-//     go to LDS as one u64 row per (z, y) in [-1, R]^2 (bits x = 0..R-1)
-//     plus one byte per row for x = -1 and x = R.  Rows of uniform chunks
-//     (and of chunks beyond the world: air) are synthesised without a read.
-//  2. face bits of a row are XORs of rows: +x = row ^ (row >> 1 | x=R bit),
-//     +y / +z = row ^ the next row.  Their popcounts give per-row counts,
+//     go to LDS as one row of R+2 bits per (z, y) in [-1, R]^2, in 32-bit
+//     words (three at R = 64).  Rows of uniform chunks (and of chunks beyond
+//     the world: air) are synthesised without a read.
+//  2. face bits of a row are XORs of rows: +x = row ^ row >> 1, +y / +z =
+//     row ^ the next row.  Their popcounts give per-row counts,
 //     per-group (8 rows at R = 64) offsets by a workgroup scan, and the
 //     chunk's face count, which is published and turned into an output
 //     offset by a decoupled look-back before any face is written.
@@ -22,11 +22,13 @@
 //  4. per pass, each thread first does everything but the stores for its
 //     faces (ambient terms from the LDS bits, the solid voxel's colour and
 //     the shadow-map entries from memory), packed into one word per face,
-//     and then only the stores: the vertex quad (32 B) and index row (24 B)
-//     of consecutive faces come from consecutive lanes.  A load issued after
-//     a store completes after it (the vector memory counter retires in
-//     order), so keeping the loads ahead of the stores keeps the stores from
-//     stalling the next face's loads.
+//     and then only the stores, shared out by address: half a vertex quad
+//     (16 of 32 B) or a third of an index row (8 of 24 B) per lane, whole
+//     lines per instruction.  A load issued after a store completes after it
+//     (the vector memory counter retires in order), so keeping the loads
+//     ahead of the stores keeps the stores from stalling the next face's
+//     loads.
+// 2048x256x2048 world, 150.3 M faces: 2985 -> 2645 us, 3.7 TB/s (the kernel).
 #include "vp_internal.h"
 
 #include <algorithm>
@@ -645,7 +647,7 @@ extern "C" int vp_gpu_mesh(vp_ctx *ctx, const vp_world_desc *world, const uint8_
     // Short lists: a chunk's face count takes a small part of its time, so
     // several workgroups repeat it and share out the faces, as many as the
     // grid holds at once and at most R / 4 (100 chunks around a camera:
-    // 358 -> 131 us).
+    // 358 -> 136 us).
     const uint32_t resident = (uint32_t)ctx->num_cus * 2u;
     a.parts = 1u;
     if (!count_only && root_bitw >= 5 && n && n <= resident / 2u)

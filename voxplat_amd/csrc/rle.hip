@@ -19,7 +19,8 @@
 // positions, set as bits of an LDS bitmap; an output byte's run is the rank of
 // the last start at or before it, so every 16-byte store is independent.
 // Bound by its stores and by the scan's latency: a 2048x256x2048 world (1.07 GB
-// of voxels from 0.2 GB of words) 547 -> 268 us, 4.8 TB/s.
+// of voxels from 0.2 GB of words) 554 -> 270 us, 4.7 TB/s (the kernel; reopening
+// the world with it, the uniform table included, 600 -> 333 us).
 #include "vp_internal.h"
 
 namespace vp {
@@ -353,7 +354,7 @@ __global__ void __launch_bounds__(BS) k_rle_decode(RleArgs a)
     // Round r hands entries r G .. r G + G - 1 to the G workgroups, rotated by a
     // golden-section step per round: with the plain stride a workgroup of a
     // whole world meets the same height every time, all air or all caves.
-    // (2048x256x2048 world: 324 -> 265 us.)
+    // (2048x256x2048 world: 324 -> 265 us, the kernel.)
     const uint32_t G = gridDim.x / a.parts, turn = (uint32_t)(0.618f * (float)G) | 1u;
     uint32_t slot = blockIdx.x / a.parts;
     // a part's share of the chunk's 16-byte pieces, in multiples of the workgroup

@@ -540,11 +540,6 @@ __device__ __forceinline__ void wave_fence()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ uint32_t ld_relaxed32(const uint32_t *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // The tile bounds of a block's box, row by row over the lanes of a wave, all
 // of whose lanes call with the same box.  The first 64 or fewer are loaded
 // ahead (box_first); more of them are read when the block is tested.
@@ -757,9 +752,10 @@ __device__ __forceinline__ bool splat_open(const uint2 rec, float lodf, const Sp
 
 // Blocks whose splats are at least this many pixels wide are handed out in
 // quarters: their sprites cost so much that a wave with a whole block of them
-// outlasts the others (15 views of 425x425 close to a 7.9 M list: 2954 against
-// 3332 us; 2422x2321: 1010 against 1190 us).  Farther blocks are cheaper whole,
-// one look at their bounds each (all of them in quarters: 1.2x the time).
+// outlasts the others (two views close to a 7.7 M list: 5870 against 9860 us at
+// 1697x1495, 13310 against 20970 at 2422x2321; to a 31 M list at 1920x1080: 4370
+// against 7620).  Farther blocks are cheaper whole, one look at their bounds each
+// (all of them in quarters: 1.2x the time).
 constexpr float kNearPixels = 5.0f;
 // Frames of up to this many pixels are rasterised without the tile bounds: the
 // whole frame stays in the L2s, and rejecting a fragment by its own load is
@@ -781,13 +777,13 @@ constexpr uint32_t kHeld = kBlock + 64;   // a wave's queue: less than a wave, a
 // full waves of them are rasterised.  Every second block a wave refreshes up to
 // kRefresh groups of its share of the tile bounds, in turn (every block or every
 // fourth: within 3%).
-// Bound by vector instructions (78% of the SIMDs' issue slots): a 1920x1080
-// frame of a 130.5 M list has 312 K blocks and 77 M splats in view, of which
-// 48% and 20% are not dropped here; each splat rasterised costs some hundred
-// instructions per 4 pixels.  1503 -> 880 us per frame against rasterising
-// every splat in view, 344 -> 275 us per 512x512 view of a 32 M list.  The
-// order's counter is not shared on purpose: an atomic ticket per block (13 ns
-// each on one address) took 1242-3786 us.
+// Bound by latency and instructions together (vector instructions fill a third of
+// the SIMDs' cycles, 1.3e8 of them a frame): a 1920x1080 frame of a 133.5 M list
+// has 297 K blocks, 76 M splats in view, of which 60% and 27% are not dropped here
+// (four worlds: 55-60%, 21-27%); each splat rasterised costs some hundred
+// instructions per 4 pixels.  1573 -> 846 us per frame (kernel) against rasterising
+// every splat in view.  The order's counter is not shared on purpose: an atomic
+// ticket per block (13 ns each on one address) took 1242-3786 us.
 __global__ void __launch_bounds__(kBlock) k_raster_blocks(const int16_t *splats,
                                                            const uint8_t *lod, uint32_t lod_log2,
                                                            uint64_t n, SplatCam c,
@@ -1370,7 +1366,7 @@ __device__ __forceinline__ uint32_t lane_up(uint32_t v)
 // Gradient of the splat colours.  Neighbouring pixels of a row mostly show the
 // same splat, so runs of one splat inside groups of 8 lanes are added up first
 // (three DPP steps) and their first lane adds the sum: the kernel is bound by
-// its atomics (a 512x512 frame: 30.2 -> 22.6 us).
+// its atomics (a 512x512 frame: 29.9 -> 22.7 us).
 __global__ void k_backward(uint64_t np, uint64_t n, const uint32_t *idbuf, const float *weight,
                            const float *dL, float *grad)
 {
